@@ -158,7 +158,7 @@ struct agx_mesh {
   agx::Arrays arr;
   bool mixed = false;                // AGX_PREC_MIXED
   bool iso = false;                  // isothermal EOS (NHYDRO = 4)
-  int tile = 5;                      // stage form of the last VL2 stage (agx_autotune; 5 = k_vl2, 32 x 8)
+  int tile = 5;                      // stage form of the last VL2 stage (default_form, agx_autotune)
   int tile1 = 5;                     // stage form of the first (donor-cell) stage
   hipStream_t stream = nullptr;
   double *pool = nullptr;            // all MHD arrays

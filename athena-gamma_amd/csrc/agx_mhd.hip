@@ -117,15 +117,57 @@ static dim3 plane_grid(int il, int iu, int jl, int ju, int kl, int ku, int nb) {
 }
 
 // Stage forms and tiles: TI x TJ (i,j) columns per workgroup of TI*TJ threads (256, or
-// 512 for the 64 x 8 tile); grid.x = tiles of one MeshBlock, grid.y = MeshBlock.  Forms
-// 0-3 run the fluxes as three k_flux launches and the rest of the stage as k_stage with
-// the tile shown; forms 4-5 run the whole stage as one k_vl2 launch.  The form is picked
-// per mesh by agx_autotune (default: 5).
-constexpr int NTILE = 6, TILE_VL2 = 4, TILE_DEFAULT = 5;
+// 512 for the 64 x 8 tile); grid.x = tiles of one MeshBlock, grid.y = chunks of k-planes,
+// grid.z = MeshBlock.  Forms 0-3 run the fluxes as k_flux launches and the rest of the
+// stage as k_stage with the tile shown; forms 4-5 run the whole stage as one k_vl2 launch.
+// The form of each stage is set by default_form, or per mesh by agx_autotune.
+constexpr int NTILE = 6, TILE_VL2 = 4;
 constexpr int TILE_I[NTILE] = {16, 32, 64, 64, 16, 32}, TILE_J[NTILE] = {16, 8, 4, 8, 16, 8};
+static int stage_tiles(const Geo &g, int tile) {
+  return ((g.bx1 + TILE_I[tile] - 1) / TILE_I[tile]) * ((g.bx2 + TILE_J[tile] - 1) / TILE_J[tile]);
+}
+
+// k-planes each workgroup of a stage kernel walks.  A workgroup that owns kc planes runs
+// kc + 1 (k_stage) or kc + 2 (k_vl2) plane iterations, so few long chunks waste least, but
+// a mesh with fewer tiles than the chip has resident workgroups (256 CUs x 4 of k_stage, 2
+// of its 512-thread tile and of k_vl2) needs its planes split to occupy it: a 64 x 32 x 32
+// block has 8 tiles, and its FP64 PLM cycle takes 1596 us with whole columns and 148 us with
+// one plane per workgroup (k_vl2 32 x 8).  The time of r resident rounds of workgroups was
+// measured (FP64 k_vl2, meshes of 64 x 32 x 32 to 256^3, 8 .. 4096 workgroups) as 0.8 of
+// one full round while half the slots are empty, 1 up to r = 1, then 0.92 r + 0.08 plus half
+// of the last round's empty share over the full rounds; the chunk count with the smallest
+// (iterations x rounds) is taken.
+static int stage_planes(const Geo &g, int tile) {
+  const double slots = (tile >= TILE_VL2 || TILE_I[tile] * TILE_J[tile] > 256) ? 512.0 : 1024.0;
+  const int extra = tile >= TILE_VL2 ? 2 : 1;
+  const double cols = (double)stage_tiles(g, tile) * g.nb;
+  int best = g.bx3;
+  double least = 0.0;
+  for (int n = 1; n <= g.bx3; ++n) {
+    const int kc = (g.bx3 + n - 1) / n;
+    const double r = cols * ((g.bx3 + kc - 1) / kc) / slots;
+    const double rounds = r <= 0.5 ? 0.8 : (r <= 1.0 ? 1.0 : 0.92 * r + 0.08 + 0.5 * (std::ceil(r) - r) / std::floor(r));
+    const double t = (kc + extra) * rounds;
+    if (n == 1 || t < least) { least = t; best = kc; }
+  }
+  return best;
+}
+
 static dim3 stage_grid(const Geo &g, int tile) {
-  int nti = (g.bx1 + TILE_I[tile] - 1) / TILE_I[tile], ntj = (g.bx2 + TILE_J[tile] - 1) / TILE_J[tile];
-  return dim3((unsigned)(nti * ntj), (unsigned)g.nb);
+  const int kc = stage_planes(g, tile);
+  return dim3((unsigned)stage_tiles(g, tile), (unsigned)((g.bx3 + kc - 1) / kc), (unsigned)g.nb);
+}
+
+// The form of a stage of reconstruction order `order` before any autotuning: the one launch
+// over 32 x 8 tiles, or the split form where that is faster: for PPM, whose faces cost
+// most (k_vl2 solves a quarter of them twice), and on meshes so small that k_vl2 would run chunks of
+// one or two planes (twice the work and more).  Cycles in us, k_vl2 against split: 64 x 32 x 32
+// 148 : 117, 64^3 in 32^3 blocks 263 : 236, 128^3 in 32^3 1369 : 1859 (FP64 PLM);
+// 120 x 90 x 70 in 40 x 30 x 14 blocks 1491 : 890 (FP64 PPM), 128^3 in 64^3 1692 : 1280 (mixed PPM).
+// Split tiles: 32 x 8 where it fits the rows (17 .. 32 cells), else 64 x 4.
+static int default_form(const Geo &g, int order) {
+  const int split = (g.bx1 > 16 && g.bx1 <= 32) ? 1 : 2;
+  return (order == 3 || stage_planes(g, 5) <= 2) ? split : 5;
 }
 
 template <typename X>
@@ -1661,10 +1703,11 @@ __device__ __forceinline__ double wg_min256(double m, double *sh) { return wg_mi
 // kernels, so results are identical.
 //
 // A workgroup owns a TI x TJ tile of (i,j) columns of one MeshBlock (thread = column) and
-// walks the cell planes upwards.  Iteration c computes the cell-centred E of plane c+1
-// and the corner EMFs of edge plane c and plane c into LDS (three planes of cell-centred
-// E, two of edges), then, after one barrier, each thread does the CT of the faces of its
-// cell in plane c-1 and of its x3 face in face plane c, and updates that cell.  Faces
+// walks kc cell planes kb .. kl upwards (stage_planes).  Iteration c computes the
+// cell-centred E of plane c+1 and the corner EMFs of edge plane c and plane c into LDS
+// (three planes of cell-centred E, two of edges), then, after one barrier, each thread does
+// the CT of the faces of its cell in plane c-1 and of its x3 face in face plane c, and
+// updates that cell.  Faces
 // shared by two cells are computed by both from identical inputs; fluxes, face EMFs and
 // weights stream from HBM once.  Outputs go to registers other than the inputs (u may
 // be in place: each cell reads only its own src), so tiles that share halo values never
@@ -1721,7 +1764,7 @@ struct StageArgs {
 // otherwise they receive the un-floored u and are converted by k_ghost_c2p.
 template <int TI, int TJ, typename TW, bool ISO, bool PUSH>
 __global__ void __launch_bounds__(TI * TJ, 4)   // >= 4 waves per SIMD: <= 128 VGPRs
-k_stage(Geo g, StageArgs<TW> a) {
+k_stage(Geo g, StageArgs<TW> a, int kc) {
   static_assert(TI * TJ == 256 || TI * TJ == 512, "k_stage runs 256- or 512-thread workgroups");
   constexpr int NH = ISO ? 4 : NHYDRO;   // conserved variables (no energy if isothermal)
   constexpr int NT = TI * TJ, CI = TI + 2, CJ = TJ + 2;
@@ -1734,7 +1777,8 @@ k_stage(Geo g, StageArgs<TW> a) {
   const int tx = tid % TI, ty = tid / TI;
   const int nti = (g.bx1 + TI - 1) / TI;
   const uint3 wg = xcd_block();   // whole MeshBlocks per XCD: tiles share halo lines in L2
-  const int b = wg.y;
+  const int b = wg.z;
+  const int kb = g.ks + (int)wg.y * kc, kl = min(kb + kc - 1, g.ke);   // cell planes of this chunk
   const int i0 = g.is + (int)(wg.x % nti) * TI;
   const int j0 = g.js + (int)(wg.x / nti) * TJ;
   const int ni = min(TI, g.ie + 1 - i0), nj = min(TJ, g.je + 1 - j0);
@@ -1763,20 +1807,20 @@ k_stage(Geo g, StageArgs<TW> a) {
       s_cce[sl][2][jj][ii] = vy * bx - vx * by;
     }
   };
-  cce_plane(g.ks - 1);
-  cce_plane(g.ks);
+  cce_plane(kb - 1);
+  cce_plane(kb);
   __syncthreads();
   double b3_lo = 0.0;       // new b3 at the lower face of cell plane c-1
   double dtmin = DBL_MAX;
-  for (int c = g.ks; c <= g.ke + 1; ++c) {
+  for (int c = kb; c <= kl + 1; ++c) {
     const int cb = c & 1, pb = cb ^ 1;
     const int cc = c % 3, pc = (c + 2) % 3;
     // (A) cell-centred E of plane c+1 (used by the next iteration), then the edges at the
     // points (c, j0+jj, i0+ii), jj in [0,nj], ii in [0,ni]: e1 and e2 of edge plane c
     // (lower edges of cell plane c; e1 for ii < ni, e2 for jj < nj) and e3 of plane c.
     // One thread per point, so weights shared by the three edges load once.
-    if (c + 1 <= g.ke + 1) cce_plane(c + 1);
-    const bool do3 = (c <= g.ke);
+    if (c + 1 <= kl + 1) cce_plane(c + 1);
+    const bool do3 = (c <= kl);
     for (int q = tid; q < np; q += NT) {
       const int jj = q / (ni + 1), ii = q - jj * (ni + 1);
       const bool do1 = ii < ni, do2 = jj < nj;
@@ -1817,15 +1861,17 @@ k_stage(Geo g, StageArgs<TW> a) {
         const double area = dx1 * dx2;
         v -= (wght / area) * (dx2 * s_e2[cb][ty][tx + 1] - dx2 * s_e2[cb][ty][tx]);
         v += (wght / area) * (dx1 * s_e1[cb][ty + 1][tx] - dx1 * s_e1[cb][ty][tx]);
-        a.d3[fo] = v;
         b3_hi = v;
-        int r[6];
-        push_range(i, g.is, g.ie, g.bx1, g.ng, r[0], r[1]);
-        push_range(j, g.js, g.je, g.bx2, g.ng, r[2], r[3]);
-        push_range(c, g.ks, g.ke + 1, g.bx3, g.ng, r[4], r[5]);
-        for_each_ghost(g, b, c, j, i, r, [&](int nb, int64_t id2) { a.d3[(int64_t)nb * S + id2] = v; });
+        if (c <= kl || c == g.ke + 1) {   // the face above the chunk is the next chunk's to write
+          a.d3[fo] = v;
+          int r[6];
+          push_range(i, g.is, g.ie, g.bx1, g.ng, r[0], r[1]);
+          push_range(j, g.js, g.je, g.bx2, g.ng, r[2], r[3]);
+          push_range(c, g.ks, g.ke + 1, g.bx3, g.ng, r[4], r[5]);
+          for_each_ghost(g, b, c, j, i, r, [&](int nb, int64_t id2) { a.d3[(int64_t)nb * S + id2] = v; });
+        }
       }
-      if (c - 1 >= g.ks) {
+      if (c - 1 >= kb) {
         const int64_t id = IDX(g, c - 1, j, i);
         const int64_t fo = fb + id;
         const double area1 = dx2 * dx3, area2 = dx1 * dx3;
@@ -1958,7 +2004,7 @@ k_stage(Geo g, StageArgs<TW> a) {
   }
   if (a.dtpart) {
     double m = wg_min<TI * TJ / 64>(dtmin, s_red);
-    if (tid == 0) a.dtpart[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = m;
+    if (tid == 0) a.dtpart[((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = m;
   }
 }
 
@@ -1973,8 +2019,8 @@ k_stage(Geo g, StageArgs<TW> a) {
 // kernels' own traffic is gone.  Every value is formed by the same operations, in the
 // same order, as the split path (k_flux + k_stage), so results are identical bit for bit.
 //
-// A workgroup owns a TI x TJ tile of (i,j) columns of one MeshBlock and walks the cell
-// planes c = ks-1 .. ke+1.  Per plane:
+// A workgroup owns a TI x TJ tile of (i,j) columns and kc cell planes kb .. kl of one
+// MeshBlock (stage_planes) and walks the planes c = kb-1 .. kl+1.  Per plane:
 //   F  faces of plane c: x1 faces i0..i0+ni of rows j0-1..j0+nj, x2 faces j0..j0+nj of
 //      columns i0-1..i0+ni, and x3 faces of face plane c (below cell plane c) of the tile
 //      and its one-cell ring without corners; then the cell-centred E of plane c.  Thread
@@ -2023,7 +2069,7 @@ __device__ __forceinline__ void flux_to_mesh(int dir, const T *f, T *out) {
 
 template <int TI, int TJ, int ORDER, int RS, typename TW, bool ISO, bool PUSH>
 __global__ void __launch_bounds__(TI * TJ, 2)   // >= 2 waves per SIMD
-k_vl2(Geo g, VL2Args<TW> a) {
+k_vl2(Geo g, VL2Args<TW> a, int kc) {
   static_assert(64 % TI == 0 && TI * TJ == 256, "k_vl2 tiles: 256 threads, rows within a wavefront");
   constexpr int NH = ISO ? 4 : NHYDRO;
   constexpr int NT = TI * TJ;
@@ -2050,7 +2096,8 @@ k_vl2(Geo g, VL2Args<TW> a) {
   const int tx = tid % TI, ty = tid / TI;
   const int nti = (g.bx1 + TI - 1) / TI;
   const uint3 wg = xcd_block();   // whole MeshBlocks per XCD: tiles share halo lines in L2
-  const int b = wg.y;
+  const int b = wg.z;
+  const int kb = g.ks + (int)wg.y * kc, kl = min(kb + kc - 1, g.ke);   // cell planes of this chunk
   const int i0 = g.is + (int)(wg.x % nti) * TI;
   const int j0 = g.js + (int)(wg.x / nti) * TJ;
   const int ni = min(TI, g.ie + 1 - i0), nj = min(TJ, g.je + 1 - j0);
@@ -2084,10 +2131,10 @@ k_vl2(Geo g, VL2Args<TW> a) {
   double b3_lo = 0.0;            // new b3 at the lower face of cell plane c-1
   double dtmin = DBL_MAX;
 
-  for (int c = g.ks - 1; c <= g.ke + 1; ++c) {
+  for (int c = kb - 1; c <= kl + 1; ++c) {
     const int cb = c & 1, pb = cb ^ 1;
     // ---- F: faces of plane c, cell-centred E of plane c
-    const bool x3 = (c >= g.ks);
+    const bool x3 = (c >= kb);
     for (int q = tid; q < ntask; q += NT) {
       int dir, ii, jj;
       if (q < 3 * NT) {
@@ -2168,8 +2215,8 @@ k_vl2(Geo g, VL2Args<TW> a) {
     }
     __syncthreads();
     // ---- E: corner EMFs of edge plane c (e1, e2) and of plane c (e3)
-    if (c >= g.ks) {
-      const bool do3 = (c <= g.ke);
+    if (c >= kb) {
+      const bool do3 = (c <= kl);
       for (int q = tid; q < np; q += NT) {
         const int jj = q / (ni + 1), ii = q - jj * (ni + 1);
         const bool do1 = ii < ni, do2 = jj < nj;
@@ -2199,22 +2246,24 @@ k_vl2(Geo g, VL2Args<TW> a) {
     __syncthreads();
     // ---- U: CT of the own x3 face of face plane c, update of the own cell of plane c-1
     double b3_hi = 0.0;
-    if (own && c >= g.ks) {
+    if (own && c >= kb) {
       {
         const int64_t fo = fb + IDX(g, c, j, i);
         double v = a.s3[fo];
         const double area = dx1 * dx2;
         v -= (wght / area) * (dx2 * s_e2[cb][ty][tx + 1] - dx2 * s_e2[cb][ty][tx]);
         v += (wght / area) * (dx1 * s_e1[cb][ty + 1][tx] - dx1 * s_e1[cb][ty][tx]);
-        a.d3[fo] = v;
         b3_hi = v;
-        int r[6];
-        push_range(i, g.is, g.ie, g.bx1, g.ng, r[0], r[1]);
-        push_range(j, g.js, g.je, g.bx2, g.ng, r[2], r[3]);
-        push_range(c, g.ks, g.ke + 1, g.bx3, g.ng, r[4], r[5]);
-        for_each_ghost(g, b, c, j, i, r, [&](int nb, int64_t id2) { a.d3[(int64_t)nb * S + id2] = v; });
+        if (c <= kl || c == g.ke + 1) {   // the face above the chunk is the next chunk's to write
+          a.d3[fo] = v;
+          int r[6];
+          push_range(i, g.is, g.ie, g.bx1, g.ng, r[0], r[1]);
+          push_range(j, g.js, g.je, g.bx2, g.ng, r[2], r[3]);
+          push_range(c, g.ks, g.ke + 1, g.bx3, g.ng, r[4], r[5]);
+          for_each_ghost(g, b, c, j, i, r, [&](int nb, int64_t id2) { a.d3[(int64_t)nb * S + id2] = v; });
+        }
       }
-      if (c - 1 >= g.ks) {
+      if (c - 1 >= kb) {
         const int64_t id = IDX(g, c - 1, j, i);
         const int64_t fo = fb + id;
         const double area1 = dx2 * dx3, area2 = dx1 * dx3;
@@ -2332,7 +2381,7 @@ k_vl2(Geo g, VL2Args<TW> a) {
     TW f1hi[5];
 #pragma unroll
     for (int n = 0; n < 5; ++n) f1hi[n] = __shfl_down(f1own[n], 1, 64);
-    if (own && c >= g.ks && c <= g.ke) {
+    if (own && c >= kb && c <= kl) {
 #pragma unroll
       for (int n = 0; n < NH; ++n) {
         const double fh = (tx == ni - 1) ? (double)s_h1e[n][ty] : (double)f1hi[n];
@@ -2370,7 +2419,7 @@ k_vl2(Geo g, VL2Args<TW> a) {
   }
   if (a.dtpart) {
     double m = wg_min<NT / 64>(dtmin, s_red);
-    if (tid == 0) a.dtpart[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = m;
+    if (tid == 0) a.dtpart[((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = m;
   }
 }
 
@@ -2647,8 +2696,6 @@ int agx_mesh_create(const agx_mesh_desc *desc, agx_mesh **out) {
   m->d = *desc;
   // CFL clamp of the VL2 integrator in 3D, time_integrator.cpp:212-215,885-896
   if (m->d.cfl > 0.5) m->d.cfl = 0.5;
-  // characteristic projection is built into the split forms only: 32 x 8 for its stage
-  if (m->d.char_proj && m->d.xorder > 1) m->tile = 1;
   Geo &g = m->g;
   g.nb1 = desc->nx1 / desc->bnx1;
   g.nb2 = desc->nx2 / desc->bnx2;
@@ -2666,6 +2713,9 @@ int agx_mesh_create(const agx_mesh_desc *desc, agx_mesh **out) {
   g.PL = g.PL > g.n3 ? g.PL : g.n3;
   g.J = g.n2 + 1;
   g.S = (int64_t)(g.n3 + 1) * g.J * g.P;
+  m->tile1 = default_form(g, 1);
+  // characteristic projection is built into the split forms only: 32 x 8 for its stage
+  m->tile = (m->d.char_proj && m->d.xorder > 1) ? 1 : default_form(g, m->d.xorder);
   // variables per array: the AGX_ARR_* set, then W2, BCC2, Q1F, Q2F, Q3F
   static const int nv[ARR_TOTAL] = {5, 5, 5, 3, 1, 1, 1, 1, 1, 1, 5, 5, 5,
                                     1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1,
@@ -2718,7 +2768,7 @@ int agx_mesh_create(const agx_mesh_desc *desc, agx_mesh **out) {
     m->dtpart_n = 0;
     for (int t = 0; t < NTILE; ++t) {
       dim3 gs = stage_grid(g, t);
-      m->dtpart_n = std::max(m->dtpart_n, (int64_t)gs.x * gs.y);
+      m->dtpart_n = std::max(m->dtpart_n, (int64_t)gs.x * gs.y * gs.z);
     }
   }
   if (e == hipSuccess) e = hipMalloc(&m->red, sizeof(double) * m->red_n);
@@ -3433,16 +3483,17 @@ extern "C++" {
 template <typename TW, bool PUSH>
 static void launch_stage_t(agx_mesh *m, int tile, const StageArgs<TW> &a, dim3 grid) {
   const Geo &g = m->g;
+  const int kc = stage_planes(g, tile);
   if (m->iso) {
-    if (tile == 1) hipLaunchKernelGGL((k_stage<32, 8, TW, true, PUSH>), grid, dim3(256), 0, m->stream, g, a);
-    else if (tile == 2) hipLaunchKernelGGL((k_stage<64, 4, TW, true, PUSH>), grid, dim3(256), 0, m->stream, g, a);
-    else if (tile == 3) hipLaunchKernelGGL((k_stage<64, 8, TW, true, PUSH>), grid, dim3(512), 0, m->stream, g, a);
-    else hipLaunchKernelGGL((k_stage<16, 16, TW, true, PUSH>), grid, dim3(256), 0, m->stream, g, a);
+    if (tile == 1) hipLaunchKernelGGL((k_stage<32, 8, TW, true, PUSH>), grid, dim3(256), 0, m->stream, g, a, kc);
+    else if (tile == 2) hipLaunchKernelGGL((k_stage<64, 4, TW, true, PUSH>), grid, dim3(256), 0, m->stream, g, a, kc);
+    else if (tile == 3) hipLaunchKernelGGL((k_stage<64, 8, TW, true, PUSH>), grid, dim3(512), 0, m->stream, g, a, kc);
+    else hipLaunchKernelGGL((k_stage<16, 16, TW, true, PUSH>), grid, dim3(256), 0, m->stream, g, a, kc);
   } else {
-    if (tile == 1) hipLaunchKernelGGL((k_stage<32, 8, TW, false, PUSH>), grid, dim3(256), 0, m->stream, g, a);
-    else if (tile == 2) hipLaunchKernelGGL((k_stage<64, 4, TW, false, PUSH>), grid, dim3(256), 0, m->stream, g, a);
-    else if (tile == 3) hipLaunchKernelGGL((k_stage<64, 8, TW, false, PUSH>), grid, dim3(512), 0, m->stream, g, a);
-    else hipLaunchKernelGGL((k_stage<16, 16, TW, false, PUSH>), grid, dim3(256), 0, m->stream, g, a);
+    if (tile == 1) hipLaunchKernelGGL((k_stage<32, 8, TW, false, PUSH>), grid, dim3(256), 0, m->stream, g, a, kc);
+    else if (tile == 2) hipLaunchKernelGGL((k_stage<64, 4, TW, false, PUSH>), grid, dim3(256), 0, m->stream, g, a, kc);
+    else if (tile == 3) hipLaunchKernelGGL((k_stage<64, 8, TW, false, PUSH>), grid, dim3(512), 0, m->stream, g, a, kc);
+    else hipLaunchKernelGGL((k_stage<16, 16, TW, false, PUSH>), grid, dim3(256), 0, m->stream, g, a, kc);
   }
 }
 
@@ -3486,34 +3537,34 @@ static void launch_stage(agx_mesh *m, int tile, int stage, double wfac, double *
 // The whole stage as one k_vl2 launch (fused form); tile 0 = 16 x 16, 1 = 32 x 8 columns.
 extern "C++" {
 template <int TI, int TJ, int ORDER, typename TW, bool ISO, bool PUSH>
-static void launch_vl2_rs(agx_mesh *m, int rs, const VL2Args<TW> &a, dim3 grid) {
+static void launch_vl2_rs(agx_mesh *m, int rs, const VL2Args<TW> &a, dim3 grid, int kc) {
   if (ISO) {
     if (rs == AGX_RSOLVER_HLLE)
-      hipLaunchKernelGGL((k_vl2<TI, TJ, ORDER, AGX_RSOLVER_HLLE, TW, ISO, PUSH>), grid, dim3(256), 0, m->stream, m->g, a);
+      hipLaunchKernelGGL((k_vl2<TI, TJ, ORDER, AGX_RSOLVER_HLLE, TW, ISO, PUSH>), grid, dim3(256), 0, m->stream, m->g, a, kc);
     else
-      hipLaunchKernelGGL((k_vl2<TI, TJ, ORDER, AGX_RSOLVER_HLLD, TW, ISO, PUSH>), grid, dim3(256), 0, m->stream, m->g, a);
+      hipLaunchKernelGGL((k_vl2<TI, TJ, ORDER, AGX_RSOLVER_HLLD, TW, ISO, PUSH>), grid, dim3(256), 0, m->stream, m->g, a, kc);
   } else {
     if (rs == AGX_RSOLVER_HLLE)
-      hipLaunchKernelGGL((k_vl2<TI, TJ, ORDER, AGX_RSOLVER_HLLE, TW, ISO, PUSH>), grid, dim3(256), 0, m->stream, m->g, a);
+      hipLaunchKernelGGL((k_vl2<TI, TJ, ORDER, AGX_RSOLVER_HLLE, TW, ISO, PUSH>), grid, dim3(256), 0, m->stream, m->g, a, kc);
     else if (rs == AGX_RSOLVER_ROE)
-      hipLaunchKernelGGL((k_vl2<TI, TJ, ORDER, AGX_RSOLVER_ROE, TW, ISO, PUSH>), grid, dim3(256), 0, m->stream, m->g, a);
+      hipLaunchKernelGGL((k_vl2<TI, TJ, ORDER, AGX_RSOLVER_ROE, TW, ISO, PUSH>), grid, dim3(256), 0, m->stream, m->g, a, kc);
     else if (rs == AGX_RSOLVER_LHLLD)
-      hipLaunchKernelGGL((k_vl2<TI, TJ, ORDER, AGX_RSOLVER_LHLLD, TW, ISO, PUSH>), grid, dim3(256), 0, m->stream, m->g, a);
+      hipLaunchKernelGGL((k_vl2<TI, TJ, ORDER, AGX_RSOLVER_LHLLD, TW, ISO, PUSH>), grid, dim3(256), 0, m->stream, m->g, a, kc);
     else
-      hipLaunchKernelGGL((k_vl2<TI, TJ, ORDER, AGX_RSOLVER_HLLD, TW, ISO, PUSH>), grid, dim3(256), 0, m->stream, m->g, a);
+      hipLaunchKernelGGL((k_vl2<TI, TJ, ORDER, AGX_RSOLVER_HLLD, TW, ISO, PUSH>), grid, dim3(256), 0, m->stream, m->g, a, kc);
   }
 }
 
 template <int TI, int TJ, typename TW, bool ISO>
-static void launch_vl2_order(agx_mesh *m, int order, const VL2Args<TW> &a, dim3 grid) {
+static void launch_vl2_order(agx_mesh *m, int order, const VL2Args<TW> &a, dim3 grid, int kc) {
   if (m->copies_state == 1) {
-    if (order == 1) launch_vl2_rs<TI, TJ, 1, TW, ISO, true>(m, m->d.rsolver, a, grid);
-    else if (order == 2) launch_vl2_rs<TI, TJ, 2, TW, ISO, true>(m, m->d.rsolver, a, grid);
-    else launch_vl2_rs<TI, TJ, 3, TW, ISO, true>(m, m->d.rsolver, a, grid);
+    if (order == 1) launch_vl2_rs<TI, TJ, 1, TW, ISO, true>(m, m->d.rsolver, a, grid, kc);
+    else if (order == 2) launch_vl2_rs<TI, TJ, 2, TW, ISO, true>(m, m->d.rsolver, a, grid, kc);
+    else launch_vl2_rs<TI, TJ, 3, TW, ISO, true>(m, m->d.rsolver, a, grid, kc);
   } else {
-    if (order == 1) launch_vl2_rs<TI, TJ, 1, TW, ISO, false>(m, m->d.rsolver, a, grid);
-    else if (order == 2) launch_vl2_rs<TI, TJ, 2, TW, ISO, false>(m, m->d.rsolver, a, grid);
-    else launch_vl2_rs<TI, TJ, 3, TW, ISO, false>(m, m->d.rsolver, a, grid);
+    if (order == 1) launch_vl2_rs<TI, TJ, 1, TW, ISO, false>(m, m->d.rsolver, a, grid, kc);
+    else if (order == 2) launch_vl2_rs<TI, TJ, 2, TW, ISO, false>(m, m->d.rsolver, a, grid, kc);
+    else launch_vl2_rs<TI, TJ, 3, TW, ISO, false>(m, m->d.rsolver, a, grid, kc);
   }
 }
 
@@ -3545,12 +3596,13 @@ static void launch_vl2(agx_mesh *m, int tile, int stage, int order, double wfac,
   a.grav = m->d.self_gravity ? 1 : 0;
   a.dtpart = dtpart;
   const dim3 grid = stage_grid(g, tile);
+  const int kc = stage_planes(g, tile);
   if (m->iso) {
-    if (tile == 5) launch_vl2_order<32, 8, TW, true>(m, order, a, grid);
-    else launch_vl2_order<16, 16, TW, true>(m, order, a, grid);
+    if (tile == 5) launch_vl2_order<32, 8, TW, true>(m, order, a, grid, kc);
+    else launch_vl2_order<16, 16, TW, true>(m, order, a, grid, kc);
   } else {
-    if (tile == 5) launch_vl2_order<32, 8, TW, false>(m, order, a, grid);
-    else launch_vl2_order<16, 16, TW, false>(m, order, a, grid);
+    if (tile == 5) launch_vl2_order<32, 8, TW, false>(m, order, a, grid, kc);
+    else launch_vl2_order<16, 16, TW, false>(m, order, a, grid, kc);
   }
 }
 }  // extern "C++"
@@ -3639,7 +3691,7 @@ static int cycle_device(agx_mesh *m) {
   if (!rc) rc = stage_fused(m, 2, true);
   if (!rc && m->d.self_gravity) rc = mg_solve(m, 2);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_min_final, dim3(1), dim3(256), 0, m->stream, m->dtpart, (int64_t)sg.x * sg.y, m->scal);
+  hipLaunchKernelGGL(k_min_final, dim3(1), dim3(256), 0, m->stream, m->dtpart, (int64_t)sg.x * sg.y * sg.z, m->scal);
   hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, m->stream, m->scal, m->d.cfl);
   LAUNCH_CHECK("k_advance");
   return 0;
@@ -3731,7 +3783,7 @@ static int cycle_segment(agx_mesh *m, int seg, int k, std::vector<MGSnap> &snaps
     return 0;
   }
   const dim3 sg = stage_grid(m->g, m->tile);
-  hipLaunchKernelGGL(k_min_final, dim3(1), dim3(256), 0, m->stream, m->dtpart, (int64_t)sg.x * sg.y, m->scal);
+  hipLaunchKernelGGL(k_min_final, dim3(1), dim3(256), 0, m->stream, m->dtpart, (int64_t)sg.x * sg.y * sg.z, m->scal);
   hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, m->stream, m->scal, m->d.cfl);
   LAUNCH_CHECK("k_advance");
   snaps.assign(1, mg_snap(m));
@@ -3850,7 +3902,7 @@ int agx_cycle(agx_mesh *m, double tlim, int32_t ncycles, int32_t *done) {
     m->time += m->dt;
     double bdt = 0.0;
     timer_begin(m, AGX_K_NEWDT);
-    rc = finish_block_dt(m, m->dtpart, (int64_t)sg.x * sg.y, &bdt);
+    rc = finish_block_dt(m, m->dtpart, (int64_t)sg.x * sg.y * sg.z, &bdt);
     timer_end(m);
     if (rc) break;
     set_new_dt(m, bdt, tlim);

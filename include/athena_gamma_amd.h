@@ -333,7 +333,8 @@ int agx_mg_levels(agx_mesh *m, int32_t *nlevels, int32_t *dims, int32_t cap);
  * fastest for each; *choice gets the second stage's form.  Forms 0..3: three flux launches, then one stage
  * kernel over 16x16, 32x8, 64x4 (i,j) columns per 256-thread workgroup or 64x8 per
  * 512-thread workgroup; forms 4..5: the whole stage (fluxes in LDS) in one launch over
- * 16x16 or 32x8 columns (form 5 is the default).  With multigrid
+ * 16x16 or 32x8 columns.  Without autotuning each stage runs form 5, or on small meshes and
+ * for PPM a split form.  With multigrid
  * gravity (periodic boundaries) it also times V-cycles with the red-black pass fused into
  * one launch and as two sweeps, and keeps the faster.  It writes only scratch registers
  * (u1, b1, fluxes, the multigrid levels, which every solve reloads), so call it between
