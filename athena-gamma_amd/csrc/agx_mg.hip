@@ -428,76 +428,6 @@ k_mg_fmg_prolong(const T *__restrict__ cu, T *__restrict__ u, int n1, int n2, in
   u[t] = acc / T(32768.0);
 }
 
-// The coarse end of a V(1,1) cycle in one workgroup: from level `top` (at most
-// COARSE_CELLS cells) down to the 1-cell level 0 (red sweep, black sweep, defect +
-// restriction per level), level 0 zeroed (SolveCoarsestGrid of a 1-cell periodic root,
-// multigrid_driver.cpp:781-787), and back up (prolongation + correction, red, black).
-// Each step is the per-cell arithmetic of k_mg_smooth, k_mg_defect_restrict and
-// k_mg_prolong, separated by workgroup barriers (which order global-memory accesses
-// within the workgroup), so the result equals the per-level launches; it replaces about
-// six launches per level.
-constexpr int COARSE_CELLS = 4096, COARSE_BS = 1024, MAXLEV = 24;
-template <typename T>
-struct CoarseLevels {
-  T *u[MAXLEV];
-  T *src[MAXLEV];
-  int n1[MAXLEV], n2[MAXLEV], n3[MAXLEV];
-  T dx2[MAXLEV], idx2[MAXLEV];
-};
-
-template <typename T>
-__device__ __forceinline__ void coarse_smooth(const CoarseLevels<T> &L, int l, int color, T isix) {
-  const int n1 = L.n1[l], n2 = L.n2[l], n3 = L.n3[l];
-  const int nh = (n1 + 1) / 2;
-  T *u = L.u[l];
-  const T *src = L.src[l];
-  for (int t = threadIdx.x; t < nh * n2 * n3; t += COARSE_BS) {
-    int h = t % nh, r = t / nh;
-    int j = r % n2, k = r / n2;
-    int i = 2 * h + ((color + k + j) & 1);
-    if (i >= n1) continue;
-    int64_t id = LIX(n1, n2, k, j, i);
-    T uc = u[id];
-    T ukp = u[LIX(n1, n2, wrapp(k, n3), j, i)], ujp = u[LIX(n1, n2, k, wrapp(j, n2), i)];
-    T uip = u[LIX(n1, n2, k, j, wrapp(i, n1))];
-    T ukm = u[LIX(n1, n2, wrapm(k, n3), j, i)], ujm = u[LIX(n1, n2, k, wrapm(j, n2), i)];
-    T uim = u[LIX(n1, n2, k, j, wrapm(i, n1))];
-    u[id] = gs_value(uc, ukp, ujp, uip, ukm, ujm, uim, src[id], L.dx2[l], isix);
-  }
-  __syncthreads();
-}
-
-template <typename T>
-__global__ void __launch_bounds__(COARSE_BS)
-k_mg_coarse(const int *__restrict__ gate, CoarseLevels<T> L, int top, int coffset, T isix, int first_sweep_done) {
-  if (gate && *gate) return;   // a closed gate: the recorded V-cycle loop has ended
-  for (int l = top; l > 0; --l) {
-    if (!(first_sweep_done && l == top)) coarse_smooth(L, l, 0 ^ coffset, isix);
-    coarse_smooth(L, l, 1 ^ coffset, isix);
-    const int c1 = L.n1[l - 1], c2 = L.n2[l - 1], c3 = L.n3[l - 1];
-    for (int t = threadIdx.x; t < c1 * c2 * c3; t += COARSE_BS) {
-      int i = t % c1, r = t / c1;
-      int j = r % c2, k = r / c2;
-      L.src[l - 1][t] = restricted_defect<T>(L.u[l], L.src[l], L.n1[l], L.n2[l], L.n3[l], k, j, i, L.idx2[l]);
-      L.u[l - 1][t] = T(0.0);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) L.u[0][0] = T(0.0);
-  __syncthreads();
-  for (int l = 1; l <= top; ++l) {
-    const int n1 = L.n1[l], n2 = L.n2[l], n3 = L.n3[l];
-    for (int t = threadIdx.x; t < n1 * n2 * n3; t += COARSE_BS) {
-      int fi = t % n1, r = t / n1;
-      int fj = r % n2, fk = r / n2;
-      L.u[l][t] += prolong_corr<T>(L.u[l - 1], L.n1[l - 1], L.n2[l - 1], L.n3[l - 1], fk, fj, fi);
-    }
-    __syncthreads();
-    coarse_smooth(L, l, 0 ^ coffset, isix);
-    coarse_smooth(L, l, 1 ^ coffset, isix);
-  }
-}
-
 // Reductions: a launch of at most NPART workgroups, workgroup w summing the contiguous
 // range [t0, t1) of the level (XCD-aware order); the partials are summed by one
 // workgroup (k_mg_final).  The order is fixed, so results are deterministic.
@@ -1069,141 +999,294 @@ k_mb_add32(const int *__restrict__ gate, double *__restrict__ u, const float *__
   u[t] += (double)e[t];
 }
 
-// The coarse end of a multipole V(1,1) cycle (vcycle_b, and vcycle_b32 in FP32) in one
-// workgroup: levels `top` (at most MB_COARSE_CELLS interior cells) down to 0 and back,
-// each step the per-element arithmetic of k_mb_bc (k_mb_bc_hom for the FP32 correction,
-// HOM), k_mb_fas, k_mb_smooth, k_mb_restrict and k_mb_prolong, separated by workgroup
-// barriers, so the potential equals the per-level launches bit for bit.  Every barrier
-// is reached by every thread: loops have workgroup-uniform bounds.
-constexpr int MB_COARSE_CELLS = 512, MB_MAXC = 8;
+// The coarse end of a V(1,1) cycle (vcycle, vcycle_b, vcycle_b32) in one workgroup: levels
+// `top` down to 0 and back, held in LDS from the first load to the last store.  Each step is
+// the per-cell arithmetic of the per-level kernels (k_mg_smooth, k_mg_defect_restrict,
+// k_mg_prolong; k_mb_fas, k_mb_smooth, k_mb_restrict, k_mb_prolong with the chain of k_mb_bc,
+// or k_mb_bc_hom for the FP32 correction), separated by workgroup barriers, so the result
+// equals the per-level launches bit for bit.  What bounds it is the latency of a step: about
+// 35 (multipole) or 24 (periodic) steps run one after the other on one CU.  Through global
+// memory the periodic levels of 16^3 and below took 28 us, from LDS 18; the multipole levels
+// of 8^3 and below took 44 us, with ghost fills between the steps, and those of 16^3 and
+// below (14 launches more) now 35.
+//
+// Framed levels keep u with its frame, where each face ghost holds the constant 2 phi_s and
+// a stencil next to it takes 2 phi_s - (its own cell), the value a ghost fill would have
+// stored; so no fills run between the steps.  The frame of (u - uold) that the prolongation
+// reads, edges and corners included, comes from the chains when the coarse level is done.
+// Every barrier is reached by every thread: loops have workgroup-uniform bounds.
+enum : int { BC_PER, BC_MP, BC_HOM };   // periodic wrap; multipole values; homogeneous chain
+constexpr int COARSE_CELLS = 4096, COARSE_BS = 1024, MAXC = 8;
+constexpr int COARSE_LDS = 15872;   // elements: 124 KB of the CU's 160 KB in FP64
+
 template <typename T>
-struct CoarseB {
-  T *u[MB_MAXC], *src[MB_MAXC], *uold[MB_MAXC];
-  const double *bcv[MB_MAXC];
-  MPGeom G[MB_MAXC];
-  double dx[MB_MAXC];
+struct CoarseLevel {
+  T *u, *src, *old;
+  const double *bcv;
+  int n1, n2, n3;
+  T dx2, idx2;
+  int lu, ls, lo, lb;   // offsets in LDS of u, src, old (below top) and bcv (below top)
 };
-template <typename T, bool HOM>
-__device__ __forceinline__ void mbc_bc(const CoarseB<T> &L, int l) {
-  const MPGeom &G = L.G[l];
-  const unsigned ng = 2u * (G.n1 + 2) * (G.n2 + 2) + 2u * G.n3 * (G.n1 + 2) + 2u * G.n3 * G.n2;
-  T *u = L.u[l];
-  for (unsigned q = threadIdx.x; q < ng; q += COARSE_BS) {
-    GhostChain c;
-    if (!ghost_chain(G, q, c)) continue;
-    T v = u[BX(G.n1, G.n2, c.kk, c.jj, c.ii)];
-    for (int d = c.depth - 1; d >= 0; --d) {
-      if (HOM) v = -v;
-      else v = 2.0 * L.bcv[l][3 * (int64_t)q + d] - v;
-    }
-    u[BX(G.n1, G.n2, c.k, c.j, c.i)] = v;
+template <typename T>
+struct CoarseSet {
+  CoarseLevel<T> lv[MAXC];
+};
+
+// t / n for t < 2^14: the quotient in FP32 is within 2^-8 / n of (t + 1/2) / n, which is at
+// least 1 / (2n) away from a whole number
+struct FastDiv {
+  float inv;
+  __device__ __forceinline__ explicit FastDiv(int n) : inv(1.0f / (float)n) {}
+  __device__ __forceinline__ int operator()(int t) const { return (int)(((float)t + 0.5f) * inv); }
+};
+
+// Ghost q of a framed level in the order of ghost_chain: its cell, the interior cell at the
+// end of its chain and the chain's length
+struct GhostCell {
+  int k, j, i, kk, jj, ii, depth;
+};
+__host__ __device__ __forceinline__ int ghost_count(int n1, int n2, int n3) {
+  return 2 * (n1 + 2) * (n2 + 2) + 2 * n3 * (n1 + 2) + 2 * n3 * n2;
+}
+__device__ __forceinline__ GhostCell ghost_cell(int n1, int n2, int n3, int q) {
+  const int w1 = n1 + 2, w2 = n2 + 2, np = 2 * w1 * w2, nr = 2 * n3 * w1;
+  GhostCell c;
+  if (q < np) {
+    const int side = q >= w1 * w2, r = q - side * w1 * w2;
+    c.k = side ? n3 + 1 : 0; c.j = FastDiv(w1)(r); c.i = r - c.j * w1;
+  } else if ((q -= np) < nr) {
+    const int row = FastDiv(w1)(q);
+    c.i = q - row * w1; c.k = 1 + row / 2; c.j = (row & 1) ? n2 + 1 : 0;
+  } else {
+    q -= nr;
+    const int row = q / 2, kr = FastDiv(n2)(row);
+    c.i = (q & 1) ? n1 + 1 : 0; c.k = 1 + kr; c.j = 1 + row - kr * n2;
   }
-  __syncthreads();
+  c.kk = min(max(c.k, 1), n3); c.jj = min(max(c.j, 1), n2); c.ii = min(max(c.i, 1), n1);
+  c.depth = (c.k != c.kk) + (c.j != c.jj) + (c.i != c.ii);
+  return c;
+}
+// the chain's value from the interior value v and its boundary values b[0 .. depth)
+template <int KIND, typename T>
+__device__ __forceinline__ T chain_value(T v, int depth, const double *b) {
+  for (int d = depth - 1; d >= 0; --d) {
+    if constexpr (KIND == BC_MP) v = 2.0 * b[d] - v;
+    else v = -v;
+  }
+  return v;
+}
+
+// u and its six neighbours at interior cell (k, j, i) of a level in LDS (0-based)
+template <typename T>
+struct Cross {
+  T c, kp, jp, ip, km, jm, im;
+};
+template <int KIND, typename T>
+__device__ __forceinline__ int coarse_id(const CoarseLevel<T> &L, int k, int j, int i) {
+  return KIND == BC_PER ? (k * L.n2 + j) * L.n1 + i : ((k + 1) * (L.n2 + 2) + j + 1) * (L.n1 + 2) + i + 1;
+}
+template <int KIND, typename T>
+__device__ __forceinline__ Cross<T> cross_at(const CoarseLevel<T> &L, const T *u, int k, int j, int i) {
+  const int n1 = L.n1, n2 = L.n2, n3 = L.n3;
+  const int id = coarse_id<KIND>(L, k, j, i);
+  Cross<T> x;
+  x.c = u[id];
+  if constexpr (KIND == BC_PER) {
+    const int sk = n1 * n2;
+    x.kp = u[k == n3 - 1 ? id - (n3 - 1) * sk : id + sk];
+    x.km = u[k == 0 ? id + (n3 - 1) * sk : id - sk];
+    x.jp = u[j == n2 - 1 ? id - (n2 - 1) * n1 : id + n1];
+    x.jm = u[j == 0 ? id + (n2 - 1) * n1 : id - n1];
+    x.ip = u[i == n1 - 1 ? id - (n1 - 1) : id + 1];
+    x.im = u[i == 0 ? id + n1 - 1 : id - 1];
+  } else {
+    const int sj = n1 + 2, sk = sj * (n2 + 2);
+    x.kp = u[id + sk]; x.km = u[id - sk];
+    x.jp = u[id + sj]; x.jm = u[id - sj];
+    x.ip = u[id + 1]; x.im = u[id - 1];
+    if (k == n3 - 1) x.kp -= x.c;
+    if (k == 0) x.km -= x.c;
+    if (j == n2 - 1) x.jp -= x.c;
+    if (j == 0) x.jm -= x.c;
+    if (i == n1 - 1) x.ip -= x.c;
+    if (i == 0) x.im -= x.c;
+  }
+  return x;
 }
 template <typename T>
-__device__ __forceinline__ void mbc_smooth(const CoarseB<T> &L, int l, int color) {
-  const int n1 = L.G[l].n1, n2 = L.G[l].n2, n3 = L.G[l].n3, nh = (n1 + 1) / 2;
-  T *u = L.u[l];
-  const T *src = L.src[l];
-  const T dx2 = T(L.dx[l] * L.dx[l]), isix = T(1.15 / 6.0);
-  for (unsigned t = threadIdx.x; t < (unsigned)nh * n2 * n3; t += COARSE_BS) {
-    const int h = t % nh, r = t / nh;
-    const int j = 1 + r % n2, k = 1 + r / n2;
-    const int i = 1 + 2 * h + ((color + k + j) & 1);
-    if (i > n1) continue;
-    const unsigned id = BX(n1, n2, k, j, i), sj = n1 + 2, sk = (unsigned)(n1 + 2) * (n2 + 2);
-    u[id] = gs_value(u[id], u[id + sk], u[id + sj], u[id + 1], u[id - sk], u[id - sj], u[id - 1], src[id], dx2,
-                     isix);
-  }
-  __syncthreads();
+__device__ __forceinline__ T cross_lap(const Cross<T> &x) {   // operand order of mb_defect / defect_at
+  return T(6.0) * x.c - x.kp - x.jp - x.ip - x.km - x.jm - x.im;
 }
-template <typename T>
-__device__ __forceinline__ void mbc_fas(const CoarseB<T> &L, int l) {
-  const int n1 = L.G[l].n1, n2 = L.G[l].n2, n3 = L.G[l].n3;
-  const unsigned w1 = n1 + 2, w2 = n2 + 2, sj = w1, sk = w1 * w2;
-  const T idx2 = T(1.0 / (L.dx[l] * L.dx[l]));
-  T *src = L.src[l], *uold = L.uold[l];
-  const T *u = L.u[l];
-  for (unsigned t = threadIdx.x; t < w1 * w2 * (unsigned)(n3 + 2); t += COARSE_BS) {
-    uold[t] = u[t];
-    const int i = t % w1, r = t / w1, j = r % w2, k = r / w2;
-    if (i < 1 || i > n1 || j < 1 || j > n2 || k < 1 || k > n3) continue;
-    src[t] -= (T(6.0) * u[t] - u[t + sk] - u[t + sj] - u[t + 1] - u[t - sk] - u[t - sj] - u[t - 1]) * idx2;
-  }
-  __syncthreads();
-}
-template <typename T>
-__device__ __forceinline__ void mbc_restrict(const CoarseB<T> &L, int l) {   // level l -> l-1
-  const int n1 = L.G[l].n1, n2 = L.G[l].n2, n3 = L.G[l].n3;
-  const int c1 = n1 >> 1, c2 = n2 >> 1, c3 = n3 >> 1;
-  const unsigned sj = n1 + 2, sk = (unsigned)(n1 + 2) * (n2 + 2);
-  const T idx2 = T(1.0 / (L.dx[l] * L.dx[l]));
-  const T *u = L.u[l], *src = L.src[l];
-  for (unsigned t = threadIdx.x; t < (unsigned)c1 * c2 * c3; t += COARSE_BS) {
-    const int i = 1 + t % c1, r = t / c1, j = 1 + r % c2, k = 1 + r / c2;
-    const int fi = 2 * i - 1, fj = 2 * j - 1, fk = 2 * k - 1;
-#define F(kk, jj, ii) BX(n1, n2, kk, jj, ii)
-    const unsigned f[8] = {F(fk, fj, fi), F(fk, fj, fi + 1), F(fk, fj + 1, fi), F(fk, fj + 1, fi + 1),
-                           F(fk + 1, fj, fi), F(fk + 1, fj, fi + 1), F(fk + 1, fj + 1, fi), F(fk + 1, fj + 1, fi + 1)};
-#undef F
-    T d[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) d[q] = mb_defect(u, src, f[q], sj, sk, idx2);
-    const unsigned c = BX(c1, c2, k, j, i);
-    L.src[l - 1][c] = T(0.125) * (d[0] + d[1] + d[2] + d[3] + d[4] + d[5] + d[6] + d[7]);
-    L.u[l - 1][c] = T(0.125) * (u[f[0]] + u[f[1]] + u[f[2]] + u[f[3]] + u[f[4]] + u[f[5]] + u[f[6]] + u[f[7]]);
-  }
-  __syncthreads();
-}
-template <typename T>
-__device__ __forceinline__ void mbc_prolong(const CoarseB<T> &L, int l) {   // level l-1 -> l
-  const int n1 = L.G[l].n1, n2 = L.G[l].n2, n3 = L.G[l].n3;
-  const int c1 = n1 >> 1, c2 = n2 >> 1;
-  const T *cu = L.u[l - 1], *cuold = L.uold[l - 1];
-  T *fu = L.u[l];
-  for (unsigned t = threadIdx.x; t < (unsigned)n1 * n2 * n3; t += COARSE_BS) {
-    const int fi = 1 + t % n1, r = t / n1, fj = 1 + r % n2, fk = 1 + r / n2;
-    const int i = (fi - 1) / 2 + 1, j = (fj - 1) / 2 + 1, k = (fk - 1) / 2 + 1;
-    const int di = ((fi - 1) & 1) ? 1 : -1, dj = ((fj - 1) & 1) ? 1 : -1, dk = ((fk - 1) & 1) ? 1 : -1;
-#define C(kk, jj, ii) (cu[BX(c1, c2, kk, jj, ii)] - cuold[BX(c1, c2, kk, jj, ii)])
-    fu[BX(n1, n2, fk, fj, fi)] +=
-        T(0.015625) * (T(27.0) * C(k, j, i) + C(k + dk, j + dj, i + di) +
-                       T(9.0) * (C(k, j, i + di) + C(k, j + dj, i) + C(k + dk, j, i)) +
-                       T(3.0) * (C(k + dk, j + dj, i) + C(k + dk, j, i + di) + C(k, j + dj, i + di)));
-#undef C
+
+template <int KIND, typename T>
+__device__ __forceinline__ void coarse_smooth(const CoarseLevel<T> &L, T *s, int color, T isix) {
+  const int nh = (L.n1 + 1) / 2;
+  const FastDiv dh(nh), d2(L.n2);
+  T *u = s + L.lu;
+  const T *src = s + L.ls;
+  for (int t = threadIdx.x; t < nh * L.n2 * L.n3; t += COARSE_BS) {
+    const int r = dh(t), k = d2(r), j = r - k * L.n2;
+    const int i = 2 * (t - r * nh) + ((color + k + j) & 1);
+    if (i >= L.n1) continue;
+    const Cross<T> x = cross_at<KIND>(L, u, k, j, i);
+    u[coarse_id<KIND>(L, k, j, i)] = gs_value(x.c, x.kp, x.jp, x.ip, x.km, x.jm, x.im,
+                                              src[(k * L.n2 + j) * L.n1 + i], L.dx2, isix);
   }
   __syncthreads();
 }
 
-template <typename T, bool HOM>
-__global__ void __launch_bounds__(COARSE_BS)
-k_mb_coarse(const int *__restrict__ gate, CoarseB<T> L, int top, int fmglevel, int coffset, int ni) {
-  if (gate && *gate) return;   // a closed gate: the recorded V-cycle loop has ended
-  for (int l = top; l > 0; --l) {
-    mbc_bc<T, HOM>(L, l);
-    if (l < fmglevel) mbc_fas(L, l);
-    mbc_smooth(L, l, 0 ^ coffset);
-    mbc_bc<T, HOM>(L, l);
-    mbc_smooth(L, l, 1 ^ coffset);
-    mbc_bc<T, HOM>(L, l);
-    mbc_restrict(L, l);
+template <int KIND, typename T>
+__device__ __forceinline__ void coarse_fas(const CoarseLevel<T> &L, T *s, T *old, const double *bcv) {
+  const FastDiv d1(L.n1), d2(L.n2);
+  const T *u = s + L.lu;
+  T *src = s + L.ls;
+  for (int t = threadIdx.x; t < L.n1 * L.n2 * L.n3; t += COARSE_BS) {
+    const int r = d1(t), i = t - r * L.n1, k = d2(r), j = r - k * L.n2;
+    const Cross<T> x = cross_at<KIND>(L, u, k, j, i);
+    old[coarse_id<KIND>(L, k, j, i)] = x.c;
+    src[t] -= cross_lap(x) * L.idx2;
   }
-  mbc_bc<T, HOM>(L, 0);
-  mbc_fas(L, 0);
-  for (int it = 0; it < ni; ++it) {
-    mbc_smooth(L, 0, 0 ^ coffset);
-    mbc_bc<T, HOM>(L, 0);
-    mbc_smooth(L, 0, 1 ^ coffset);
-    mbc_bc<T, HOM>(L, 0);
+  for (int q = threadIdx.x; q < ghost_count(L.n1, L.n2, L.n3); q += COARSE_BS) {
+    const GhostCell c = ghost_cell(L.n1, L.n2, L.n3, q);
+    old[BX(L.n1, L.n2, c.k, c.j, c.i)] = chain_value<KIND>(u[BX(L.n1, L.n2, c.kk, c.jj, c.ii)], c.depth, bcv + 3 * q);
+  }
+  __syncthreads();
+}
+
+template <int KIND, typename T>
+__device__ __forceinline__ void coarse_restrict(const CoarseLevel<T> &F, const CoarseLevel<T> &C, T *s) {
+  const FastDiv d1(C.n1), d2(C.n2);
+  const T *u = s + F.lu, *src = s + F.ls;
+  for (int t = threadIdx.x; t < C.n1 * C.n2 * C.n3; t += COARSE_BS) {
+    const int r = d1(t), i = t - r * C.n1, k = d2(r), j = r - k * C.n2;
+    T sd = T(0.0), su = T(0.0);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int fk = 2 * k + (q >> 2), fj = 2 * j + ((q >> 1) & 1), fi = 2 * i + (q & 1);
+      const Cross<T> x = cross_at<KIND>(F, u, fk, fj, fi);
+      const T d = cross_lap(x) * F.idx2 + src[(fk * F.n2 + fj) * F.n1 + fi];
+      sd = q ? sd + d : d;
+      su = q ? su + x.c : x.c;
+    }
+    s[C.ls + t] = T(0.125) * sd;
+    s[C.lu + coarse_id<KIND>(C, k, j, i)] = KIND == BC_PER ? T(0.0) : T(0.125) * su;
+  }
+  __syncthreads();
+}
+
+// old = u - old over the framed level (the values k_mb_prolong interpolates)
+template <int KIND, typename T>
+__device__ __forceinline__ void coarse_change(const CoarseLevel<T> &L, T *s, const double *bcv) {
+  const FastDiv d1(L.n1), d2(L.n2);
+  const T *u = s + L.lu;
+  T *old = s + L.lo;
+  for (int t = threadIdx.x; t < L.n1 * L.n2 * L.n3; t += COARSE_BS) {
+    const int r = d1(t), k = d2(r), id = coarse_id<KIND>(L, k, r - k * L.n2, t - r * L.n1);
+    old[id] = u[id] - old[id];
+  }
+  for (int q = threadIdx.x; q < ghost_count(L.n1, L.n2, L.n3); q += COARSE_BS) {
+    const GhostCell c = ghost_cell(L.n1, L.n2, L.n3, q);
+    const unsigned id = BX(L.n1, L.n2, c.k, c.j, c.i);
+    old[id] = chain_value<KIND>(u[BX(L.n1, L.n2, c.kk, c.jj, c.ii)], c.depth, bcv + 3 * q) - old[id];
+  }
+  __syncthreads();
+}
+
+template <int KIND, typename T>
+__device__ __forceinline__ void coarse_prolong(const CoarseLevel<T> &F, const CoarseLevel<T> &C, T *s) {
+  const FastDiv d1(F.n1), d2(F.n2);
+  T *u = s + F.lu;
+  const T *c = s + (KIND == BC_PER ? C.lu : C.lo);
+  for (int t = threadIdx.x; t < F.n1 * F.n2 * F.n3; t += COARSE_BS) {
+    const int r = d1(t), fi = t - r * F.n1, fk = d2(r), fj = r - fk * F.n2;
+    const int i = fi >> 1, j = fj >> 1, k = fk >> 1;
+    int ip = i + ((fi & 1) ? 1 : -1), jp = j + ((fj & 1) ? 1 : -1), kp = k + ((fk & 1) ? 1 : -1);
+    if constexpr (KIND == BC_PER) { ip = wrap(ip, C.n1); jp = wrap(jp, C.n2); kp = wrap(kp, C.n3); }
+#define V(kk, jj, ii) c[coarse_id<KIND>(C, kk, jj, ii)]
+    u[coarse_id<KIND>(F, fk, fj, fi)] +=
+        T(0.015625) * (T(27.0) * V(k, j, i) + V(kp, jp, ip) + T(9.0) * (V(k, j, ip) + V(k, jp, i) + V(kp, j, i)) +
+                       T(3.0) * (V(kp, jp, i) + V(kp, j, ip) + V(k, jp, ip)));
+#undef V
+  }
+  __syncthreads();
+}
+
+template <typename T, int KIND>
+__global__ void __launch_bounds__(COARSE_BS)
+k_mg_coarse(const int *__restrict__ gate, CoarseSet<T> S, int top, int fmglevel, int coffset, int ni, T isix,
+            int first_sweep_done) {
+  if (gate && *gate) return;   // a closed gate: the recorded V-cycle loop has ended
+  __shared__ T s[COARSE_LDS];
+  {
+    const CoarseLevel<T> &L = S.lv[top];
+    const FastDiv d1(L.n1), d2(L.n2);
+    for (int t = threadIdx.x; t < L.n1 * L.n2 * L.n3; t += COARSE_BS) {
+      const int r = d1(t), k = d2(r), id = coarse_id<KIND>(L, k, r - k * L.n2, t - r * L.n1);
+      s[L.lu + id] = L.u[id];
+      s[L.ls + t] = L.src[KIND == BC_PER ? t : id];
+    }
+  }
+  if constexpr (KIND != BC_PER) {
+    for (int l = 0; l <= top; ++l) {
+      const CoarseLevel<T> &L = S.lv[l];
+      for (int q = threadIdx.x; q < ghost_count(L.n1, L.n2, L.n3); q += COARSE_BS) {
+        const GhostCell c = ghost_cell(L.n1, L.n2, L.n3, q);
+        T face = T(0.0);
+        if constexpr (KIND == BC_MP) {
+          face = 2.0 * L.bcv[3 * q];
+          if (l < top)
+            for (int d = 0; d < c.depth; ++d) s[L.lb + 3 * q + d] = L.bcv[3 * q + d];
+        }
+        s[L.lu + BX(L.n1, L.n2, c.k, c.j, c.i)] = face;   // read at face ghosts only
+      }
+    }
+  }
+  __syncthreads();
+  // boundary values of level l: in LDS below top (T is double with multipole values)
+  auto bv = [&](int l) -> const double * {
+    if constexpr (KIND == BC_MP) return l < top ? s + S.lv[l].lb : S.lv[l].bcv;
+    else return nullptr;
+  };
+  for (int l = top; l > 0; --l) {
+    if constexpr (KIND != BC_PER)
+      if (l < fmglevel) coarse_fas<KIND>(S.lv[l], s, l < top ? s + S.lv[l].lo : S.lv[l].old, bv(l));
+    if (!(first_sweep_done && l == top)) coarse_smooth<KIND>(S.lv[l], s, 0 ^ coffset, isix);
+    coarse_smooth<KIND>(S.lv[l], s, 1 ^ coffset, isix);
+    coarse_restrict<KIND>(S.lv[l], S.lv[l - 1], s);
+  }
+  if constexpr (KIND == BC_PER) {   // SolveCoarsestGrid of the one-cell root, multigrid_driver.cpp:781-787
+    if (threadIdx.x == 0) s[S.lv[0].lu] = T(0.0);
+    __syncthreads();
+  } else {
+    coarse_fas<KIND>(S.lv[0], s, 0 < top ? s + S.lv[0].lo : S.lv[0].old, bv(0));
+    for (int it = 0; it < ni; ++it) {
+      coarse_smooth<KIND>(S.lv[0], s, 0 ^ coffset, isix);
+      coarse_smooth<KIND>(S.lv[0], s, 1 ^ coffset, isix);
+    }
   }
   for (int l = 1; l <= top; ++l) {
-    mbc_bc<T, HOM>(L, l - 1);
-    mbc_prolong(L, l);
-    mbc_bc<T, HOM>(L, l);
-    mbc_smooth(L, l, 0 ^ coffset);
-    mbc_bc<T, HOM>(L, l);
-    mbc_smooth(L, l, 1 ^ coffset);
-    mbc_bc<T, HOM>(L, l);
+    if constexpr (KIND != BC_PER) coarse_change<KIND>(S.lv[l - 1], s, bv(l - 1));
+    coarse_prolong<KIND>(S.lv[l], S.lv[l - 1], s);
+    coarse_smooth<KIND>(S.lv[l], s, 0 ^ coffset, isix);
+    coarse_smooth<KIND>(S.lv[l], s, 1 ^ coffset, isix);
+  }
+  // u of every level (a later solve may start from it), with top's frame filled
+  for (int l = 0; l <= top; ++l) {
+    const CoarseLevel<T> &L = S.lv[l];
+    const FastDiv d1(L.n1), d2(L.n2);
+    for (int t = threadIdx.x; t < L.n1 * L.n2 * L.n3; t += COARSE_BS) {
+      const int r = d1(t), k = d2(r), id = coarse_id<KIND>(L, k, r - k * L.n2, t - r * L.n1);
+      L.u[id] = s[L.lu + id];
+    }
+  }
+  if constexpr (KIND != BC_PER) {
+    const CoarseLevel<T> &L = S.lv[top];
+    const double *b = bv(top);
+    for (int q = threadIdx.x; q < ghost_count(L.n1, L.n2, L.n3); q += COARSE_BS) {
+      const GhostCell c = ghost_cell(L.n1, L.n2, L.n3, q);
+      L.u[BX(L.n1, L.n2, c.k, c.j, c.i)] =
+          chain_value<KIND>(s[L.lu + BX(L.n1, L.n2, c.kk, c.jj, c.ii)], c.depth, b + 3 * q);
+    }
   }
 }
 
@@ -1522,51 +1605,79 @@ static void fas_b(agx_mesh *m, int l) {
   timer_end(m);
 }
 
-// SolveVCycle(1,1) (multigrid_driver.cpp:684-693) with the FAS steps of
-// OneStepToCoarser / SolveCoarsestGrid / OneStepToFiner (:583-677, :778-819) and the
-// MeshBlock task lists (mg_task_list.cpp:258-262, 287-510).  Boundaries are filled before
-// every stencil step, as the reference's exchanges and ApplyPhysicalBoundaries are.
-// Highest level k_mb_coarse takes (at most MB_COARSE_CELLS interior cells, at most
-// MB_MAXC levels from 0), or -1 when switched off (agx_set_mg_coarse)
-static int coarse_top_b(const agx_mesh *m) {
-  if (!m->mg_coarse) return -1;
-  int top = -1;
-  for (int l = 0; l < m->ntotal && l < MB_MAXC; ++l) {
-    const MGLevelB &B = m->levb[l];
-    if ((int64_t)B.n1 * B.n2 * B.n3 <= MB_COARSE_CELLS) top = l;
+// Highest level k_mg_coarse takes: at most COARSE_CELLS interior cells, levels 0 .. top within
+// its LDS; -1 if there is none.  N1 .. N3 from the level list, framed or not.
+template <typename LV>
+static int coarse_lds(const std::vector<LV> &H, int top, bool framed, bool bcv) {   // LDS elements
+  int64_t n = 0;
+  for (int l = 0; l <= top; ++l) {
+    const LV &L = H[l];
+    const int64_t c = (int64_t)L.n1 * L.n2 * L.n3, f = (int64_t)(L.n1 + 2) * (L.n2 + 2) * (L.n3 + 2);
+    n += framed ? f + c : 2 * c;
+    if (framed && l < top) n += f + (bcv ? 3 * (f - c) : 0);
   }
+  return (int)std::min<int64_t>(n, INT32_MAX);
+}
+template <typename LV>
+static int coarse_fit(const std::vector<LV> &H, bool framed, bool bcv) {
+  int top = -1;
+  while (top + 1 < (int)H.size() && top + 1 < MAXC &&
+         (int64_t)H[top + 1].n1 * H[top + 1].n2 * H[top + 1].n3 <= COARSE_CELLS &&
+         coarse_lds(H, top + 1, framed, bcv) <= COARSE_LDS)
+    ++top;
   return top;
 }
+template <typename T, typename LV>
+static CoarseSet<T> coarse_set(const std::vector<LV> &H, int top, bool framed, bool bcv) {
+  CoarseSet<T> S = {};
+  int o = 0;
+  for (int l = 0; l <= top; ++l) {
+    const LV &L = H[l];
+    CoarseLevel<T> &c = S.lv[l];
+    c.u = L.u;
+    c.src = L.src;
+    c.n1 = L.n1; c.n2 = L.n2; c.n3 = L.n3;
+    c.dx2 = T(L.dx * L.dx);
+    c.idx2 = T(1.0 / (L.dx * L.dx));
+    const int n = L.n1 * L.n2 * L.n3, f = (L.n1 + 2) * (L.n2 + 2) * (L.n3 + 2);
+    c.lu = o; o += framed ? f : n;
+    c.ls = o; o += n;
+    if (framed && l < top) {
+      c.lo = o; o += f;
+      if (bcv) { c.lb = o; o += 3 * (f - n); }
+    }
+  }
+  return S;
+}
+
+static int coarse_top_b(const agx_mesh *m) { return m->mg_coarse ? coarse_fit(m->levb, true, true) : -1; }
 
 static void coarse_b(agx_mesh *m, int top, int ni) {
-  CoarseB<double> c;
+  CoarseSet<double> c = coarse_set<double>(m->levb, top, true, true);
   for (int l = 0; l <= top; ++l) {
-    MGLevelB &B = m->levb[l];
-    c.u[l] = B.u; c.src[l] = B.src; c.uold[l] = B.uold; c.bcv[l] = B.bcv;
-    c.G[l] = mp_geom(m, B);
-    c.dx[l] = B.dx;
+    c.lv[l].old = m->levb[l].uold;
+    c.lv[l].bcv = m->levb[l].bcv;
   }
   timer_begin(m, AGX_K_MG_OTHER);
-  hipLaunchKernelGGL((k_mb_coarse<double, false>), dim3(1), dim3(COARSE_BS), 0, m->stream, m->gate, c, top, m->fmglevel,
-                     m->coffset, ni);
+  hipLaunchKernelGGL((k_mg_coarse<double, BC_MP>), dim3(1), dim3(COARSE_BS), 0, m->stream, m->gate, c, top,
+                     m->fmglevel, m->coffset, ni, 1.15 / 6.0, 0);
   timer_end(m);
 }
 
 // the same for the FP32 correction cycle (homogeneous boundary chain)
 static void coarse_b32(agx_mesh *m, int top, int ni) {
-  CoarseB<float> c;
-  for (int l = 0; l <= top; ++l) {
-    MGLevelB32 &B = m->levb32[l];
-    c.u[l] = B.u; c.src[l] = B.src; c.uold[l] = B.uold; c.bcv[l] = nullptr;
-    c.G[l] = mp_geom(m, m->levb[l]);
-    c.dx[l] = B.dx;
-  }
+  CoarseSet<float> c = coarse_set<float>(m->levb32, top, true, false);
+  for (int l = 0; l <= top; ++l) c.lv[l].old = m->levb32[l].uold;
   timer_begin(m, AGX_K_MG_OTHER);
-  hipLaunchKernelGGL((k_mb_coarse<float, true>), dim3(1), dim3(COARSE_BS), 0, m->stream, m->gate, c, top, m->fmglevel,
-                     m->coffset, ni);
+  hipLaunchKernelGGL((k_mg_coarse<float, BC_HOM>), dim3(1), dim3(COARSE_BS), 0, m->stream, m->gate, c, top,
+                     m->fmglevel, m->coffset, ni, float(1.15 / 6.0), 0);
   timer_end(m);
 }
 
+// SolveVCycle(1,1) (multigrid_driver.cpp:684-693) with the FAS steps of
+// OneStepToCoarser / SolveCoarsestGrid / OneStepToFiner (:583-677, :778-819) and the
+// MeshBlock task lists (mg_task_list.cpp:258-262, 287-510).  Boundaries are filled before
+// every stencil step, as the reference's exchanges and ApplyPhysicalBoundaries are.
 static void vcycle_b(agx_mesh *m) {
   int start = m->current;
   m->coffset ^= 1;
@@ -2179,27 +2290,17 @@ static void solve_coarsest(agx_mesh *m, std::vector<MGLevelT<T>> &H) {
 // black.
 // Highest level handled by k_mg_coarse, or -1 if the root grid is not a single cell.
 template <typename T>
-static int coarse_top(agx_mesh *m, const std::vector<MGLevelT<T>> &H) {
+static int coarse_top(const std::vector<MGLevelT<T>> &H) {
   const MGLevelT<T> &L0 = H[0];
-  if (L0.n1 != 1 || L0.n2 != 1 || L0.n3 != 1 || (int)H.size() > MAXLEV) return -1;
-  int top = 0;
-  while (top + 1 < (int)H.size() && lcells(H[top + 1]) <= COARSE_CELLS) ++top;
-  return top;
+  return (L0.n1 == 1 && L0.n2 == 1 && L0.n3 == 1) ? coarse_fit(H, false, false) : -1;
 }
 
 template <typename T>
 static void coarse_cycle(agx_mesh *m, std::vector<MGLevelT<T>> &H, int top, bool first_sweep_done) {
-  CoarseLevels<T> c;
-  for (int l = 0; l <= top; ++l) {
-    c.u[l] = H[l].u;
-    c.src[l] = H[l].src;
-    c.n1[l] = H[l].n1; c.n2[l] = H[l].n2; c.n3[l] = H[l].n3;
-    c.dx2[l] = T(H[l].dx * H[l].dx);
-    c.idx2[l] = T(1.0 / (H[l].dx * H[l].dx));
-  }
   timer_begin(m, AGX_K_MG_SMOOTH);
-  hipLaunchKernelGGL(k_mg_coarse<T>, dim3(1), dim3(COARSE_BS), 0, m->stream, m->gate, c, top, m->coffset,
-                     T(1.15 / 6.0), first_sweep_done ? 1 : 0);
+  hipLaunchKernelGGL((k_mg_coarse<T, BC_PER>), dim3(1), dim3(COARSE_BS), 0, m->stream, m->gate,
+                     coarse_set<T>(H, top, false, false), top, 0, m->coffset, 0, T(1.15 / 6.0),
+                     first_sweep_done ? 1 : 0);
   timer_end(m);
 }
 
@@ -2207,7 +2308,7 @@ template <typename T>
 static void vcycle(agx_mesh *m, std::vector<MGLevelT<T>> &H, bool first_sweep_done = false) {
   int start = m->current;
   m->coffset ^= 1;
-  const int ct = coarse_top(m, H);
+  const int ct = coarse_top(H);
   while (m->current > 0 && m->current > ct) {
     int l = m->current;
     if (first_sweep_done && l == start) smooth(m, H, l, 1);

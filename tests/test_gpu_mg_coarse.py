@@ -1,0 +1,56 @@
+"""k_mg_coarse against the per-level steps at the edges of its range: the whole hierarchy in the
+kernel (16^3 cells, and one 8^3 block), the largest level it takes, root grids that are odd or
+flat, and levels just above it; the same potential bit for bit."""
+import numpy as np
+import pytest
+
+from oracle.orc import make_desc
+from tests.test_gpu_mg_levels import vcycle_by_steps
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [((8, 8, 8), 8), ((16, 16, 16), 8), ((24, 8, 8), 8), ((12, 20, 4), 4), ((64, 8, 4), 4), ((32, 32, 32), 8)]
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("n,b", SHAPES)
+def test_multipole_vcycles_identical(agx, n, b, precision):
+    """one launch against one launch per step (a mixed V-cycle is a defect-correction step)"""
+    h = 1.0 / max(n)
+    d = make_desc(nx=n, bnx=(b, b, b), box=tuple((-0.5 * h * q, 0.5 * h * q) for q in n), self_gravity=1, mg_bc=1,
+                  mg_mode=0, four_pi_G=1.0, mporder=4, mg_threshold=-1.0, mg_niter=2, precision=precision)
+    U = np.zeros((5, n[2], n[1], n[0]))
+    U[0] = np.random.default_rng(3).uniform(0.5, 1.5, n[::-1])
+    ub = agx.scatter_cells(d, U)
+    out = []
+    for on in (1, 0):
+        m = agx.Mesh(d)
+        m.set("u", ub)
+        m.set_mg_coarse(on)
+        m.mg_solve(0)
+        m.mg_solve(0)   # FMG starts from what the first solve left on the root level
+        out.append((m.get("phi"), m.mg_last()))
+        m.close()
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
+
+
+@pytest.mark.parametrize("n,b", [(8, 8), (16, 8), (16, 16), (32, 16)])
+def test_periodic_vcycle_identical(agx, n, b):
+    d = make_desc(nx=(n,) * 3, bnx=(b,) * 3, box=((0.0, 1.0),) * 3, self_gravity=1, mg_bc=0, mg_mode=0, four_pi_G=1.0,
+                  mg_threshold=-1.0, mg_niter=1)
+    U = np.zeros((5, n, n, n))
+    U[0] = np.random.default_rng(4).uniform(0.5, 1.5, (n, n, n))
+    ub = agx.scatter_cells(d, U)
+    a, c = agx.Mesh(d), agx.Mesh(d)
+    for m in (a, c):
+        m.set("u", ub)
+        m.mg_solve(0)
+    a.mg_vcycles(2)
+    for _ in range(2):
+        vcycle_by_steps(c, False)
+    assert a.mg_defect_norm() == c.mg_defect_norm()
+    for m in (a, c):
+        m.mg_step("retrieve")
+    assert np.array_equal(a.get("phi"), c.get("phi"))
+    a.close()
+    c.close()
