@@ -107,6 +107,7 @@ struct MGLevelB {
   double dx;               // cell size of the smoother/defect (as MGLevel::dx)
   double h[3];             // cell size per direction for coordinates: (xmax - xmin) / n
   double *u, *src, *uold;
+  double *tmp = nullptr, *rhs = nullptr;   // whole passes: u between the way down and the way up; FAS right-hand side
   double *bcv;             // multipole boundary values of each ghost's chain (3 per ghost)
 };
 
@@ -116,6 +117,7 @@ struct MGLevelB32 {
   int n1, n2, n3;
   double dx;
   float *u, *src, *uold;
+  float *tmp = nullptr, *rhs = nullptr;
 };
 
 // Device state of a threshold solve whose V-cycle loop is recorded for a fixed number of
@@ -128,7 +130,7 @@ struct MGGate {
 };
 
 // Host-side multigrid state that a V-cycle changes: the red-black offset, the level
-// cursor and the arrays the fused pass and the mixed correction swap.
+// cursor and the arrays the mixed correction swaps.
 struct MGSnap {
   std::vector<MGLevel> lev;
   std::vector<MGLevel32> lev32;
@@ -187,12 +189,12 @@ struct agx_mesh {
   int mg_on = 0;
   int nrootlevel = 0, nmblevel = 0, ntotal = 0, current = 0, fmglevel = 0, coffset = 0;
   int mg_mode = 0, mg_niter = 0;
-  int mg_fuse = -1;
-  int mg_coarse = 1;   // multipole V-cycles: the coarse levels in one workgroup (k_mg_coarse)
+  int mg_fuse = -1;    // periodic V-cycles: 0 one launch per step, else whole passes
+  int mg_coarse = 1;   // multipole V-cycles: coarse levels in one workgroup (k_mg_coarse), the others as whole passes
   // source mask (agx_mg_set_source_mask_sphere): src = 0 where |x - c|^2 > r^2
   int srcmask = 0;
   double srcmask_c[3] = {0.0, 0.0, 0.0};
-  double srcmask_r2 = 0.0;                  // red-black pass form: -1 by level size, 0 two sweeps, 1 fused
+  double srcmask_r2 = 0.0;
   double mg_eps = -1.0, last_norm = 0.0, last_ave = 0.0;
   int32_t last_iters = 0;
   agx::MGGate *gatedev = nullptr;    // gate of a recorded threshold loop (device)

@@ -112,109 +112,6 @@ k_mg_smooth_pairs(const int *__restrict__ gate, T *__restrict__ u, const T *__re
   u2[row + h] = c;
 }
 
-// Both sweeps of one red-black pass (red = colour c0 first, then black) in one launch:
-// reads uin, writes uout, so every red update sees the old black values and every black
-// update the new red ones, as two in-place sweeps do.  A workgroup owns a TI x TJ tile
-// of (i,j) columns and a chunk of KC planes, walking the planes upwards: it keeps the
-// old values of three planes of (tile + 2-cell ring) and the new red values of three
-// planes of (tile + 1-cell ring) in LDS, and writes plane q-1 of its tile (red copied,
-// black updated) after computing the red values of plane q.  Red cells of the ring and
-// of the planes just outside the chunk are recomputed by every workgroup that needs
-// them, from the same inputs.  Periodic wrap in all directions; every extent even.
-// Arithmetic: gs_value, the operands of k_mg_smooth.
-constexpr int RB_TI = 64, RB_TJ = 8, RB_KC = 16;
-template <typename T>
-__global__ void __launch_bounds__(RB_TI * RB_TJ)
-k_mg_smooth_rb(const int *__restrict__ gate,
-               const T *__restrict__ uin, T *__restrict__ uout, const T *__restrict__ src, int n1, int n2,
-               int n3, T dx2, T isix, int c0) {
-  if (gate && *gate) return;   // a closed gate: the recorded V-cycle loop has ended
-  constexpr int TI = RB_TI, TJ = RB_TJ, NT = TI * TJ, OI = TI + 4, OJ = TJ + 4, RI = TI + 2, RJ = TJ + 2;
-  __shared__ T s_old[3][OJ][OI];
-  __shared__ T s_red[3][RJ][RI];
-  const int tid = threadIdx.x;
-  const int nti = n1 / TI, ntj = n2 / TJ;
-  const unsigned wg = xcd_slot(blockIdx.x, gridDim.x);
-  const int tile = wg % (unsigned)(nti * ntj), chunk = wg / (unsigned)(nti * ntj);
-  const int i0 = (tile % nti) * TI, j0 = (tile / nti) * TJ;
-  const int k0 = chunk * RB_KC, k1 = min(k0 + RB_KC, n3);   // black/written planes [k0, k1)
-  auto slot = [](int q) { return ((q % 3) + 3) % 3; };
-  auto wr = [](int a, int n) { return a < 0 ? a + n : (a >= n ? a - n : a); };
-  auto load_old = [&](int q) {
-    const int kq = wr(q, n3), sl = slot(q);
-    for (int t = tid; t < OI * OJ; t += NT) {
-      const int jj = t / OI, ii = t - jj * OI;
-      s_old[sl][jj][ii] = uin[LIX(n1, n2, kq, wr(j0 - 2 + jj, n2), wr(i0 - 2 + ii, n1))];
-    }
-  };
-  auto red_plane = [&](int q) {
-    const int kq = wr(q, n3), so = slot(q), sm = slot(q - 1), sp = slot(q + 1);
-    for (int t = tid; t < RI * RJ; t += NT) {
-      const int jj = t / RI, ii = t - jj * RI;
-      const int gj = wr(j0 - 1 + jj, n2), gi = wr(i0 - 1 + ii, n1);
-      if ((gi + gj + kq + c0) & 1) continue;   // black cell
-      s_red[so][jj][ii] = gs_value(s_old[so][jj + 1][ii + 1], s_old[sp][jj + 1][ii + 1], s_old[so][jj + 2][ii + 1],
-                                   s_old[so][jj + 1][ii + 2], s_old[sm][jj + 1][ii + 1], s_old[so][jj][ii + 1],
-                                   s_old[so][jj + 1][ii], src[LIX(n1, n2, kq, gj, gi)], dx2, isix);
-    }
-  };
-  auto black_plane = [&](int q) {   // q in [k0, k1): writes the tile of plane q
-    const int so = slot(q), sm = slot(q - 1), sp = slot(q + 1);
-    for (int t = tid; t < NT; t += NT) {
-      const int jj = t / TI, ii = t - jj * TI;
-      const int gj = j0 + jj, gi = i0 + ii;
-      const int64_t id = LIX(n1, n2, q, gj, gi);
-      T v;
-      if (((gi + gj + q + c0) & 1) == 0) {
-        v = s_red[so][jj + 1][ii + 1];
-      } else {
-        v = gs_value(s_old[so][jj + 2][ii + 2], s_red[sp][jj + 1][ii + 1], s_red[so][jj + 2][ii + 1],
-                     s_red[so][jj + 1][ii + 2], s_red[sm][jj + 1][ii + 1], s_red[so][jj][ii + 1],
-                     s_red[so][jj + 1][ii], src[id], dx2, isix);
-      }
-      uout[id] = v;
-    }
-  };
-  // the old values of plane q+1 are fetched into registers one iteration ahead, so their
-  // latency overlaps the red and black updates of the previous iteration
-  constexpr int NPF = (OI * OJ + NT - 1) / NT;
-  T pf[NPF];
-  auto fetch = [&](int q) {
-    const int kq = wr(q, n3);
-#pragma unroll
-    for (int r = 0; r < NPF; ++r) {
-      const int t = tid + r * NT;
-      if (t < OI * OJ) {
-        const int jj = t / OI, ii = t - jj * OI;
-        pf[r] = uin[LIX(n1, n2, kq, wr(j0 - 2 + jj, n2), wr(i0 - 2 + ii, n1))];
-      }
-    }
-  };
-  auto stash = [&](int q) {
-    const int sl = slot(q);
-#pragma unroll
-    for (int r = 0; r < NPF; ++r) {
-      const int t = tid + r * NT;
-      if (t < OI * OJ) {
-        const int jj = t / OI, ii = t - jj * OI;
-        s_old[sl][jj][ii] = pf[r];
-      }
-    }
-  };
-  load_old(k0 - 2);
-  load_old(k0 - 1);
-  fetch(k0);
-  for (int q = k0 - 1; q <= k1; ++q) {
-    stash(q + 1);
-    if (q + 2 <= k1 + 1) fetch(q + 2);
-    __syncthreads();
-    red_plane(q);
-    __syncthreads();
-    if (q - 1 >= k0) black_plane(q - 1);
-    __syncthreads();
-  }
-}
-
 template <typename T>
 __device__ __forceinline__ T defect_at(const T *u, const T *src, int n1, int n2,
                                        int n3, int k, int j, int i, T idx2) {
@@ -551,7 +448,7 @@ k_mg_defect_to32(const int *__restrict__ gate,
 }
 
 // k_mg_defect_to32 for levels with n1 % DT_TI == 0 and n2 % DT_TJ == 0, tiled like
-// k_mg_smooth_rb: a workgroup owns a DT_TI x DT_TJ tile of (i,j) columns and a chunk of
+// k_mg_down: a workgroup owns a DT_TI x DT_TJ tile of (i,j) columns and a chunk of
 // DT_KC planes, and keeps phi (= u + e) of three planes of (tile + 1-cell ring) in LDS,
 // the next plane being fetched into registers while the current one is processed, so
 // u and e are read about once instead of seven times.  Per cell the arithmetic is that
@@ -1215,29 +1112,81 @@ template <typename T, int KIND>
 __global__ void __launch_bounds__(COARSE_BS)
 k_mg_coarse(const int *__restrict__ gate, CoarseSet<T> S, int top, int fmglevel, int coffset, int ni, T isix,
             int first_sweep_done) {
-  if (gate && *gate) return;   // a closed gate: the recorded V-cycle loop has ended
+  const int closed = gate ? *gate : 0;   // a closed gate: the recorded V-cycle loop has ended
   __shared__ T s[COARSE_LDS];
+  // every global value into registers before the first is used: the interior of top, and with
+  // multipole values its face constants and the boundary values of the levels below (the
+  // chunks that a cubic hierarchy has; loops take the rest)
+  constexpr int NI = COARSE_CELLS / COARSE_BS, NG = 2, NL = KIND == BC_MP ? 4 : 1;
+  const CoarseLevel<T> &LT = S.lv[top];
+  const int nt = LT.n1 * LT.n2 * LT.n3, gt = KIND == BC_PER ? 0 : ghost_count(LT.n1, LT.n2, LT.n3);
+  T uv[NI], sv[NI], gv[NG];
+  double bl[NL][NG];
+  int ut[NI];
   {
-    const CoarseLevel<T> &L = S.lv[top];
-    const FastDiv d1(L.n1), d2(L.n2);
-    for (int t = threadIdx.x; t < L.n1 * L.n2 * L.n3; t += COARSE_BS) {
-      const int r = d1(t), k = d2(r), id = coarse_id<KIND>(L, k, r - k * L.n2, t - r * L.n1);
-      s[L.lu + id] = L.u[id];
-      s[L.ls + t] = L.src[KIND == BC_PER ? t : id];
+    const FastDiv d1(LT.n1), d2(LT.n2);
+#pragma unroll
+    for (int e = 0; e < NI; ++e) {
+      const int t = threadIdx.x + e * COARSE_BS;
+      if (t >= nt) continue;
+      const int r = d1(t), k = d2(r);
+      ut[e] = coarse_id<KIND>(LT, k, r - k * LT.n2, t - r * LT.n1);
+      uv[e] = LT.u[ut[e]];
+      sv[e] = LT.src[KIND == BC_PER ? t : ut[e]];
+    }
+    if constexpr (KIND == BC_MP) {
+#pragma unroll
+      for (int e = 0; e < NG; ++e) {
+        const int q = threadIdx.x + e * COARSE_BS;
+        gv[e] = q < gt ? 2.0 * LT.bcv[3 * q] : 0.0;
+      }
+#pragma unroll
+      for (int l = 0; l < NL; ++l) {
+        if (l >= top) break;
+        const int nb = 3 * ghost_count(S.lv[l].n1, S.lv[l].n2, S.lv[l].n3);
+#pragma unroll
+        for (int e = 0; e < NG; ++e) {
+          const int q = threadIdx.x + e * COARSE_BS;
+          if (q < nb) bl[l][e] = S.lv[l].bcv[q];
+        }
+      }
     }
   }
-  if constexpr (KIND != BC_PER) {
+  if (closed) return;
+#pragma unroll
+  for (int e = 0; e < NI; ++e) {
+    const int t = threadIdx.x + e * COARSE_BS;
+    if (t >= nt) continue;
+    s[LT.lu + ut[e]] = uv[e];
+    s[LT.ls + t] = sv[e];
+  }
+  if constexpr (KIND == BC_MP) {
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+      if (l >= top) break;
+      const int nb = 3 * ghost_count(S.lv[l].n1, S.lv[l].n2, S.lv[l].n3);
+#pragma unroll
+      for (int e = 0; e < NG; ++e) {
+        const int q = threadIdx.x + e * COARSE_BS;
+        if (q < nb) s[S.lv[l].lb + q] = bl[l][e];
+      }
+    }
+    for (int l = 0; l < top; ++l) {
+      const int nb = 3 * ghost_count(S.lv[l].n1, S.lv[l].n2, S.lv[l].n3);
+      for (int q = threadIdx.x + (l < NL ? NG * COARSE_BS : 0); q < nb; q += COARSE_BS)
+        s[S.lv[l].lb + q] = S.lv[l].bcv[q];
+    }
+    __syncthreads();
+  }
+  if constexpr (KIND != BC_PER) {   // 2 phi_s into the face ghosts (the other ghosts are not read)
     for (int l = 0; l <= top; ++l) {
       const CoarseLevel<T> &L = S.lv[l];
-      for (int q = threadIdx.x; q < ghost_count(L.n1, L.n2, L.n3); q += COARSE_BS) {
+      for (int q = threadIdx.x, e = 0; q < ghost_count(L.n1, L.n2, L.n3); q += COARSE_BS, ++e) {
         const GhostCell c = ghost_cell(L.n1, L.n2, L.n3, q);
         T face = T(0.0);
-        if constexpr (KIND == BC_MP) {
-          face = 2.0 * L.bcv[3 * q];
-          if (l < top)
-            for (int d = 0; d < c.depth; ++d) s[L.lb + 3 * q + d] = L.bcv[3 * q + d];
-        }
-        s[L.lu + BX(L.n1, L.n2, c.k, c.j, c.i)] = face;   // read at face ghosts only
+        if constexpr (KIND == BC_MP)
+          face = l < top ? 2.0 * s[L.lb + 3 * q] : (e == 0 ? gv[0] : (e == 1 ? gv[1] : 2.0 * L.bcv[3 * q]));
+        s[L.lu + BX(L.n1, L.n2, c.k, c.j, c.i)] = face;
       }
     }
   }
@@ -1287,6 +1236,415 @@ k_mg_coarse(const int *__restrict__ gate, CoarseSet<T> S, int top, int fmglevel,
       L.u[BX(L.n1, L.n2, c.k, c.j, c.i)] =
           chain_value<KIND>(s[L.lu + BX(L.n1, L.n2, c.kk, c.jj, c.ii)], c.depth, b + 3 * q);
     }
+  }
+}
+
+// ================================================================ whole passes of a level
+// k_mg_down does everything of one level on the way down (FAS right-hand side, both sweeps,
+// restriction) and k_mg_up everything on the way up (prolongation and correction, both
+// sweeps) in one launch each; the per-step form takes three to seven, every one of them a trip
+// of the level through memory and, on small levels, 3.5 us of launch.  Every value is formed
+// by the arithmetic of the per-step kernels, so the result equals theirs bit for bit.
+//
+// A workgroup owns TP_I x TP_J columns and kc planes.  A thread owns a pair of cells along i of
+// the tile or of its ring (as wide as the steps reach) and walks the planes upwards with the
+// steps staggered: red on plane q, black on q-1, the defect on q-2.  A colour's update is one
+// cell of every pair, so no lane idles; its neighbours along k are the thread's own registers,
+// those along i and j come from the plane in LDS, updated in place.  The steps of an iteration
+// work on different planes, and one barrier a plane suffices.  256^3 FP64 periodic: 133 us down
+// (two sweeps and the restriction: 238) and 136 us up (263), where the bytes of u and source
+// alone take 80; 64^3 multipole: 14 us down and 12 up (29 and 32 with the ghost fills).  On
+// large levels an iteration's instructions bound it (about 300 for a pair of cells and a plane,
+// 44 of them floating point), on small ones their latency: loads two or three planes ahead and
+// planes split by cell parity in LDS made it no faster.  A tile held whole in LDS takes the same
+// time on small levels and 36 us instead of 34 at 128^3.
+//
+// Passes run out of place, u -> tmp on the way down and tmp -> u on the way up, as tiles read
+// each other's old values.  Periodic levels wrap; framed levels hold 2 phi_s in their face
+// ghosts, as k_mg_coarse does, and k_mg_up stores the frame that the next level's prolongation
+// and the defect sum read, k_mg_down the frame of the FAS copy.
+constexpr int TP_I = 32, TP_J = 16;
+
+template <typename T>
+struct PassArgs {
+  const T *uin;          // u (down) or tmp (up)
+  T *uout;               // tmp (down) or u (up)
+  const T *src;
+  T *rhs, *old;          // down with FAS: right-hand side and copy of u
+  T *csrc, *cu;          // down: the coarse source and u
+  const T *cc, *ccold;   // up: the coarse u and its FAS copy (framed levels)
+  const double *bcv;     // boundary values of this level (BC_MP)
+  int n1, n2, n3, kc;
+  T dx2, idx2, isix;
+  int c0;                // colour of the first sweep
+  int first_sweep_done;  // down: the first sweep is in uin already
+};
+
+template <int KIND>
+__device__ __forceinline__ int64_t pass_id(int n1, int n2, int k, int j, int i) {   // 0-based cell
+  if constexpr (KIND == BC_PER) return LIX(n1, n2, k, j, i);
+  else return (int64_t)BX(n1, n2, k + 1, j + 1, i + 1);
+}
+
+// ghost_cell's q of framed cell (k, j, i), one of its coordinates at least in the frame
+__device__ __forceinline__ unsigned ghost_index(int n1, int n2, int n3, int k, int j, int i) {
+  const unsigned w1 = n1 + 2, w2 = n2 + 2, np = 2 * w1 * w2, nr = 2 * n3 * w1;
+  if (k == 0 || k == n3 + 1) return (k ? w1 * w2 : 0) + j * w1 + i;
+  if (j == 0 || j == n2 + 1) return np + (2 * (k - 1) + (j ? 1 : 0)) * w1 + i;
+  return np + nr + 2 * ((unsigned)(k - 1) * n2 + j - 1) + (i ? 1 : 0);
+}
+
+// the ghosts whose chain ends at boundary cell (k, j, i) (0-based; every extent at least 2)
+template <int KIND, typename T>
+__device__ __forceinline__ void push_frame(T *u, const double *bcv, int n1, int n2, int n3, int k, int j, int i, T v) {
+  const int gk = k == 0 ? 0 : (k == n3 - 1 ? n3 + 1 : -1), gj = j == 0 ? 0 : (j == n2 - 1 ? n2 + 1 : -1),
+            gi = i == 0 ? 0 : (i == n1 - 1 ? n1 + 1 : -1);
+  if (gk < 0 && gj < 0 && gi < 0) return;
+  for (int e = 1; e < 8; ++e) {
+    if (((e & 4) && gk < 0) || ((e & 2) && gj < 0) || ((e & 1) && gi < 0)) continue;
+    const int kk = (e & 4) ? gk : k + 1, jj = (e & 2) ? gj : j + 1, ii = (e & 1) ? gi : i + 1;
+    const double *b = KIND == BC_MP ? bcv + 3 * (int64_t)ghost_index(n1, n2, n3, kk, jj, ii) : nullptr;
+    u[BX(n1, n2, kk, jj, ii)] = chain_value<KIND>(v, __popc(e), b);
+  }
+}
+
+// two neighbouring values, 8 bytes aligned in FP64: framed rows start at odd cells
+template <typename T>
+struct alignas(sizeof(T)) Pair {
+  T x, y;
+};
+
+// A thread's pair of columns (i, i+1), j of a tile with a ring of 2 PR cells along i and RJ
+// along j, and the plane steps on it
+template <int KIND, int PR, int RJ, typename T>
+struct PassColumn {
+  static constexpr int NP = TP_I / 2 + 2 * PR, NJ = TP_J + 2 * RJ, W = 2 * NP, PL = NJ * W;
+  static constexpr int NT = (NP * NJ + 63) / 64 * 64;
+  const PassArgs<T> &a;
+  int i0, j0, k0, ni, nj, k1;   // the tile: first cells, sizes, planes [k0, k1)
+  int p, row, i, j;             // the pair's place in the region and its first cell
+  bool in, upd, tile;           // inside the domain; a row that is updated (not the region's edge); in the tile
+  int last;                     // cells 1 .. last of a row of the region are updated
+  int near0;                    // the pair's place in LDS, its row kept off the region's edge
+  int64_t base, sk;             // index of the pair in plane 0 (wrapped), plane stride
+  __device__ __forceinline__ PassColumn(const PassArgs<T> &a_) : a(a_) {
+    const int ti = (a.n1 + TP_I - 1) / TP_I, tj = (a.n2 + TP_J - 1) / TP_J;
+    const int w = (int)xcd_slot(blockIdx.x, gridDim.x), r = w / ti;
+    i0 = (w - r * ti) * TP_I; j0 = (r % tj) * TP_J; k0 = (r / tj) * a.kc;
+    ni = min(TP_I, a.n1 - i0); nj = min(TP_J, a.n2 - j0); k1 = min(k0 + a.kc, a.n3);
+    row = (int)threadIdx.x / NP; p = (int)threadIdx.x - row * NP;
+    i = i0 - 2 * PR + 2 * p; j = j0 - RJ + row;
+    const bool use = 2 * p < ni + 4 * PR && row < nj + 2 * RJ;
+    in = use && (KIND == BC_PER || ((unsigned)j < (unsigned)a.n2 && (unsigned)i < (unsigned)a.n1));
+    upd = in && row >= 1 && row < nj + 2 * RJ - 1;
+    last = ni + 4 * PR - 2;
+    near0 = min(max(row, 1), NJ - 2) * W + 2 * p;
+    tile = use && p >= PR && 2 * p < ni + 2 * PR && row >= RJ && row < nj + RJ;
+    const int wi = KIND == BC_PER ? wrap(i, a.n1) : i, wj = KIND == BC_PER ? wrap(j, a.n2) : j;
+    base = pass_id<KIND>(a.n1, a.n2, 0, wj, wi);
+    sk = KIND == BC_PER ? (int64_t)a.n1 * a.n2 : (int64_t)(a.n1 + 2) * (a.n2 + 2);
+  }
+  __device__ __forceinline__ int plane(int q) const { return KIND == BC_PER ? wrap(q, a.n3) : q; }
+  __device__ __forceinline__ bool plane_in(int q) const { return KIND == BC_PER || (unsigned)q < (unsigned)a.n3; }
+  // plane q of x, and half the value of face ghosts (scale doubles it where it is used)
+  __device__ __forceinline__ Pair<T> load(const T *__restrict__ x, int q) const {
+    Pair<T> v = {T(0.0), T(0.0)};
+    if (in && plane_in(q)) {
+      v = *reinterpret_cast<const Pair<T> *>(x + base + plane(q) * sk);
+    } else if constexpr (KIND == BC_MP) {
+      const bool jin = (unsigned)j < (unsigned)a.n2, iin = (unsigned)i < (unsigned)a.n1, kin = plane_in(q);
+      const bool kg = q == -1 || q == a.n3, jg = j == -1 || j == a.n2;
+      if ((kg && jin && iin) || (kin && jg && iin)) {
+        const double *b = a.bcv + 3 * (int64_t)ghost_index(a.n1, a.n2, a.n3, q + 1, j + 1, i + 1);
+        v.x = b[0];
+        v.y = b[3];
+      } else if (kin && jin && i == -2) {
+        v.y = a.bcv[3 * (int64_t)ghost_index(a.n1, a.n2, a.n3, q + 1, j + 1, 0)];
+      } else if (kin && jin && i == a.n1) {
+        v.x = a.bcv[3 * (int64_t)ghost_index(a.n1, a.n2, a.n3, q + 1, j + 1, a.n1 + 1)];
+      }
+    }
+    return v;
+  }
+  __device__ __forceinline__ T scale(int q) const { return (KIND == BC_MP && !(in && plane_in(q))) ? T(2.0) : T(1.0); }
+  __device__ __forceinline__ Pair<T> load_src(const T *__restrict__ x, int q) const {
+    Pair<T> v = {T(0.0), T(0.0)};
+    if (in && plane_in(q)) v = *reinterpret_cast<const Pair<T> *>(x + base + plane(q) * sk);
+    return v;
+  }
+  // The neighbours in LDS (the row of plane s) of the pair's first (odd = 0) or second cell.
+  // Every thread reads, from a row inside the region, so that the reads of all the steps of an
+  // iteration are in flight together; the values of edge threads go nowhere.
+  struct Near {
+    T jp, jm, e;   // e: the cell beyond the pair
+  };
+  // the cell of the pair that has this colour on plane q (tiles and pairs start at even cells)
+  __device__ __forceinline__ int odd_of(int q, int color) const { return (color + q + j) & 1; }
+  __device__ __forceinline__ Near near(const T *s, int odd) const {
+    const T *t = s + near0 + odd;
+    return {t[W], t[-W], s[near0 + (odd ? 2 : -1)]};
+  }
+  // the cross of that cell on plane q: values c, neighbours along k in kp and km
+  __device__ __forceinline__ Cross<T> cross(const Near &n, const Pair<T> &c, const Pair<T> &kp, const Pair<T> &km, int q,
+                                            int odd) const {
+    Cross<T> x;
+    x.c = odd ? c.y : c.x;
+    x.kp = odd ? kp.y : kp.x;
+    x.km = odd ? km.y : km.x;
+    x.jp = n.jp;
+    x.jm = n.jm;
+    x.ip = odd ? n.e : c.y;
+    x.im = odd ? c.x : n.e;
+    if constexpr (KIND != BC_PER) {
+      if (q == a.n3 - 1) x.kp -= x.c;
+      if (q == 0) x.km -= x.c;
+      if (j == a.n2 - 1) x.jp -= x.c;
+      if (j == 0) x.jm -= x.c;
+      if (i + odd == a.n1 - 1) x.ip -= x.c;
+      if (i + odd == 0) x.im -= x.c;
+    }
+    return x;
+  }
+  // one colour on plane q, whose values are c here and s in LDS
+  __device__ __forceinline__ void smooth(T *s, const Near &n, Pair<T> &c, const Pair<T> &kp, const Pair<T> &km,
+                                         const Pair<T> &f, int q, int odd) const {
+    const Cross<T> x = cross(n, c, kp, km, q, odd);
+    const T v = gs_value(x.c, x.kp, x.jp, x.ip, x.km, x.jm, x.im, odd ? f.y : f.x, a.dx2, a.isix);
+    const int e = 2 * p + odd;
+    if (upd && e >= 1 && e <= last && plane_in(q)) {
+      if (odd) c.y = v;
+      else c.x = v;
+      s[row * W + e] = v;
+    }
+  }
+  __device__ __forceinline__ void put(T *s, const Pair<T> &v) const {
+    if (row < NJ) {
+      s[row * W + 2 * p] = v.x;
+      s[row * W + 2 * p + 1] = v.y;
+    }
+  }
+};
+
+template <typename T, int KIND, bool FAS>
+__global__ void __launch_bounds__((PassColumn<KIND, 2, 3, T>::NT))
+k_mg_down(const int *__restrict__ gate, PassArgs<T> a) {
+  const int closed = gate ? *gate : 0;   // a closed gate: the recorded V-cycle loop has ended
+  using Col = PassColumn<KIND, 2, 3, T>;
+  // planes in flight: the defect's q-2 .. q+1 (with FAS one more, as a plane's right-hand side is
+  // formed from old values before its first colour changes), and the one being stored
+  constexpr int AH = FAS ? 2 : 1, NB = 4 + AH;
+  __shared__ T s_u[NB][Col::PL];
+  __shared__ T s_d[2][TP_J][TP_I];
+  const Col t(a);
+  const int qa = t.k0 - 2, qe = t.k1 + 1;   // red planes
+  int slot = 0;                             // of plane q
+  auto buf = [&](int d) -> T * {            // plane q + d
+    int z = slot + d;
+    z = z < 0 ? z + NB : (z >= NB ? z - NB : z);
+    return s_u[z];
+  };
+  // registers: u of planes q+AH .. q-3, the source of q+1 (FAS) .. q-2, and the loads ahead
+  Pair<T> m1 = t.load(a.uin, qa - 1), c = t.load(a.uin, qa), p1 = t.load(a.uin, qa + 1), p2 = {};
+  Pair<T> f0 = t.load_src(a.src, qa), f1 = {}, fm1 = {}, fm2 = {}, m2 = {}, m3 = {};
+  if constexpr (FAS) { p2 = t.load(a.uin, qa + 2); f1 = t.load_src(a.src, qa + 1); }
+  Pair<T> un = t.load(a.uin, qa + AH + 1), fn = t.load_src(a.src, qa + AH);
+  if (closed) return;
+  auto doubled = [&](Pair<T> &v, int q) {
+    if constexpr (KIND == BC_MP) { v.x *= t.scale(q); v.y *= t.scale(q); }
+  };
+  doubled(m1, qa - 1); doubled(c, qa); doubled(p1, qa + 1);
+  t.put(buf(-1), m1);
+  t.put(buf(0), c);
+  t.put(buf(1), p1);
+  if constexpr (FAS) { doubled(p2, qa + 2); t.put(buf(2), p2); }
+  __syncthreads();
+  // FAS right-hand side of plane q (values v, neighbours up and lo) into f
+  auto fas = [&](Pair<T> &f, const T *s, const Pair<T> &v, const Pair<T> &up, const Pair<T> &lo, int q) {
+    const typename Col::Near n0 = t.near(s, 0), n1 = t.near(s, 1);
+    const T fx = f.x - cross_lap(t.cross(n0, v, up, lo, q, 0)) * a.idx2;
+    const T fy = f.y - cross_lap(t.cross(n1, v, up, lo, q, 1)) * a.idx2;
+    if (!t.plane_in(q)) return;
+    f.x = fx;
+    f.y = fy;
+    if (t.tile && q >= t.k0 && q < t.k1) {
+      *reinterpret_cast<Pair<T> *>(a.rhs + t.base + q * t.sk) = f;
+      *reinterpret_cast<Pair<T> *>(a.old + t.base + q * t.sk) = v;
+      if constexpr (KIND != BC_PER) {
+        push_frame<KIND>(a.old, a.bcv, a.n1, a.n2, a.n3, q, t.j, t.i, v.x);
+        push_frame<KIND>(a.old, a.bcv, a.n1, a.n2, a.n3, q, t.j, t.i + 1, v.y);
+      }
+    }
+  };
+  if constexpr (FAS) {
+    fas(f0, buf(0), c, p1, m1, qa);
+    __syncthreads();   // red on plane qa changes what its neighbours' right-hand sides read
+  }
+  T acc = T(0.0), uacc = T(0.0);
+  Pair<T> dl = {};   // the own pair's defects of the plane before
+  const int dj = t.row - 3, di = 2 * t.p - 4;
+  const bool even = t.tile && (dj & 1) == 0;
+  const T *const so = &s_d[0][t.tile ? dj | 1 : 0][t.tile ? di : 0];
+  for (int q = qa; q <= qe; ++q) {
+    const int odd = t.odd_of(q, a.c0), kd = q - 2, kr = q - 3;   // black on q-1 is the same cell of the pair
+    const T *s2 = buf(-2);
+    const typename Col::Near nr = t.near(buf(0), odd), nb = t.near(buf(-1), odd), d0 = t.near(s2, 0), d1 = t.near(s2, 1);
+    const Pair<T> o = {so[(kr & 1) * (TP_I * TP_J)], so[(kr & 1) * (TP_I * TP_J) + 1]};
+    if constexpr (FAS) fas(f1, buf(1), p1, p2, c, q + 1);
+    if (!a.first_sweep_done) t.smooth(buf(0), nr, c, p1, m1, f0, q, odd);
+    if (q - 1 >= t.k0 - 1) t.smooth(buf(-1), nb, m1, c, m2, fm1, q - 1, odd);
+    // restriction of plane q-3, whose defects all rows have stored; the sums run over the cells
+    // in the order of k_mg_defect_restrict / k_mb_restrict
+    acc = (kr & 1) ? acc + dl.x : dl.x;
+    acc = acc + dl.y;
+    acc = acc + o.x;
+    acc = acc + o.y;
+    if (even && kr >= t.k0 && (kr & 1)) {
+      const int64_t id = pass_id<KIND>(a.n1 >> 1, a.n2 >> 1, kr >> 1, t.j >> 1, t.i >> 1);
+      a.csrc[id] = T(0.125) * acc;
+      a.cu[id] = KIND == BC_PER ? T(0.0) : T(0.125) * uacc;
+    }
+    dl.x = cross_lap(t.cross(d0, m2, m1, m3, kd, 0)) * a.idx2 + fm2.x;
+    dl.y = cross_lap(t.cross(d1, m2, m1, m3, kd, 1)) * a.idx2 + fm2.y;
+    if constexpr (KIND != BC_PER) {
+      uacc = (kd & 1) ? uacc + m2.x : m2.x;
+      uacc = uacc + m2.y;
+      uacc = uacc + d0.jp;
+      uacc = uacc + d1.jp;
+    }
+    if (t.tile && kd >= t.k0) {
+      s_d[kd & 1][dj][di] = dl.x;
+      s_d[kd & 1][dj][di + 1] = dl.y;
+      *reinterpret_cast<Pair<T> *>(a.uout + t.base + kd * t.sk) = m2;
+    }
+    // the next plane: registers move down, the oldest slot takes plane q+AH+1
+    const int qn = q + AH + 1;
+    doubled(un, qn);
+    m3 = m2; m2 = m1; m1 = c; c = p1;
+    fm2 = fm1; fm1 = f0;
+    if constexpr (FAS) { p1 = p2; p2 = un; f0 = f1; f1 = fn; }
+    else { p1 = un; f0 = fn; }
+    t.put(buf(AH + 1 - NB), un);
+    un = t.load(a.uin, min(qn + 1, t.k1 + 2));
+    fn = t.load_src(a.src, min(q + AH + 1, t.k1 + 1));
+    slot = slot + 1 == NB ? 0 : slot + 1;
+    __syncthreads();
+  }
+  if (even) {   // the last plane (odd)
+    acc = acc + dl.x;
+    acc = acc + dl.y;
+    acc = acc + so[TP_I * TP_J];
+    acc = acc + so[TP_I * TP_J + 1];
+    const int64_t id = pass_id<KIND>(a.n1 >> 1, a.n2 >> 1, (t.k1 - 1) >> 1, t.j >> 1, t.i >> 1);
+    a.csrc[id] = T(0.125) * acc;
+    a.cu[id] = KIND == BC_PER ? T(0.0) : T(0.125) * uacc;
+  }
+}
+
+template <typename T, int KIND>
+__global__ void __launch_bounds__((PassColumn<KIND, 1, 2, T>::NT))
+k_mg_up(const int *__restrict__ gate, PassArgs<T> a) {
+  const int closed = gate ? *gate : 0;   // a closed gate: the recorded V-cycle loop has ended
+  using Col = PassColumn<KIND, 1, 2, T>;
+  constexpr int NB = 4, CI = TP_I / 2 + 4, CJ = TP_J / 2 + 4;   // coarse tile and two cells
+  static_assert(CI * CJ <= Col::NT, "one coarse cell per thread");
+  __shared__ T s_u[NB][Col::PL];
+  __shared__ T s_c[4][CJ * CI];   // u - uold (framed) or u of coarse planes, slot = plane & 3
+  const Col t(a);
+  const int c1 = a.n1 >> 1, c2 = a.n2 >> 1, c3 = a.n3 >> 1;
+  const int qa = t.k0 - 1, qe = t.k1;   // red planes
+  int slot = 0;
+  auto buf = [&](int d) -> T * {
+    int z = slot + d;
+    z = z < 0 ? z + NB : (z >= NB ? z - NB : z);
+    return s_u[z];
+  };
+  // the coarse cell this thread carries into LDS
+  const int cr = (int)threadIdx.x / CI, cj = (t.j0 >> 1) - 2 + cr, ci = (t.i0 >> 1) - 2 + (int)threadIdx.x - cr * CI;
+  const bool cuse = cr < CJ && 2 * cr < t.nj + 8 && 2 * ((int)threadIdx.x - cr * CI) < t.ni + 8;
+  auto cload = [&](int k, T &v, T &o) {
+    v = o = T(0.0);
+    if (!cuse) return;
+    k = min(k, (t.k1 >> 1) + 1);   // the last that is read
+    if constexpr (KIND == BC_PER) {
+      v = a.cc[LIX(c1, c2, wrap(k, c3), wrap(cj, c2), wrap(ci, c1))];
+    } else if (k >= -1 && k <= c3 && cj >= -1 && cj <= c2 && ci >= -1 && ci <= c1) {
+      const unsigned id = BX(c1, c2, k + 1, cj + 1, ci + 1);
+      v = a.cc[id];
+      o = a.ccold[id];
+    }
+  };
+  auto cput = [&](int k, const T &v, const T &o) {
+    if (cr < CJ) s_c[k & 3][threadIdx.x] = KIND == BC_PER ? v : v - o;
+  };
+  // plane f of the corrected u; the low child of a coarse cell leans on the cell below, the high on
+  // the one above (region parity is cell parity)
+  const int cq = ((t.row >> 1) + 1) * CI + t.p + 1, cjo = (t.row & 1) ? CI : -CI;
+  auto correct = [&](Pair<T> &v, int f) {
+    if (!t.in || !t.plane_in(f)) return;
+    const T *k0 = s_c[(f >> 1) & 3] + cq, *kn = s_c[((f >> 1) + ((f & 1) ? 1 : -1)) & 3] + cq;
+    const T C0 = k0[0], Cj = k0[cjo], Ck = kn[0], Cjk = kn[cjo];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int d = h ? 1 : -1;
+      const T Ci = k0[d], Cij = k0[cjo + d], Cik = kn[d], Cijk = kn[cjo + d];
+      (h ? v.y : v.x) += T(0.015625) * (T(27.0) * C0 + Cijk + T(9.0) * (Ci + Cj + Ck) + T(3.0) * (Cjk + Cik + Cij));
+    }
+  };
+  auto doubled = [&](Pair<T> &v, int q) {
+    if constexpr (KIND == BC_MP) { v.x *= t.scale(q); v.y *= t.scale(q); }
+  };
+  // the first red plane qa = k0 - 1 is odd: fine planes qa-1 .. qa+1 lean on coarse planes
+  // k0/2 - 2 .. k0/2, and later even planes f bring coarse plane f/2 + 1
+  const int kc0 = (t.k0 >> 1) - 2;
+  T cv[4], co[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) cload(kc0 + e, cv[e], co[e]);
+  Pair<T> m1 = t.load(a.uin, qa - 1), c = t.load(a.uin, qa), p1 = t.load(a.uin, qa + 1), m2 = {}, fm1 = {};
+  Pair<T> f0 = t.load_src(a.src, qa), un = t.load(a.uin, qa + 2), fn = t.load_src(a.src, qa + 1);
+  if (closed) return;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) cput(kc0 + e, cv[e], co[e]);
+  __syncthreads();
+  doubled(m1, qa - 1); correct(m1, qa - 1);
+  doubled(c, qa); correct(c, qa);
+  doubled(p1, qa + 1); correct(p1, qa + 1);
+  t.put(buf(-1), m1);
+  t.put(buf(0), c);
+  t.put(buf(1), p1);
+  T nv, no;   // the coarse plane after the newest
+  cload(kc0 + 4, nv, no);
+  __syncthreads();
+  for (int q = qa; q <= qe; ++q) {
+    // the plane that enters next, q+2, leans on coarse planes up to (q+3)/2, in LDS since the
+    // last barrier
+    const int f = q + 2, odd = t.odd_of(q, a.c0);
+    const typename Col::Near nr = t.near(buf(0), odd), nb = t.near(buf(-1), odd);
+    doubled(un, f);
+    if (q < qe) correct(un, f);
+    t.smooth(buf(0), nr, c, p1, m1, f0, q, odd);
+    const int kb = q - 1;
+    if (kb >= t.k0) {
+      t.smooth(buf(-1), nb, m1, c, m2, fm1, kb, odd);
+      if (t.tile) {
+        *reinterpret_cast<Pair<T> *>(a.uout + t.base + kb * t.sk) = m1;
+        if constexpr (KIND != BC_PER) {
+          push_frame<KIND>(a.uout, a.bcv, a.n1, a.n2, a.n3, kb, t.j, t.i, m1.x);
+          push_frame<KIND>(a.uout, a.bcv, a.n1, a.n2, a.n3, kb, t.j, t.i + 1, m1.y);
+        }
+      }
+    }
+    if (q == qe) break;
+    t.put(buf(2), un);
+    if ((f & 1) == 0) {   // the odd planes from f+1 on lean on coarse plane f/2 + 1
+      cput((f >> 1) + 1, nv, no);
+      cload((f >> 1) + 2, nv, no);
+    }
+    m2 = m1; m1 = c; c = p1; p1 = un;
+    fm1 = f0; f0 = fn;
+    un = t.load(a.uin, min(f + 1, t.k1 + 1));
+    fn = t.load_src(a.src, min(q + 2, t.k1));
+    slot = slot + 1 == NB ? 0 : slot + 1;
+    __syncthreads();
   }
 }
 
@@ -1528,7 +1886,7 @@ static int mp_create(agx_mesh *m) {
     B.h[0] = (m->d.x1max - m->d.x1min) / B.n1;
     B.h[1] = (m->d.x2max - m->d.x2min) / B.n2;
     B.h[2] = (m->d.x3max - m->d.x3min) / B.n3;
-    tot += 3 * pad32(bcells(B)) + pad32(3 * bghosts(B));
+    tot += (l < L - 1 ? 5 : 4) * pad32(bcells(B)) + pad32(3 * bghosts(B));
   }
   AGX_HIP(hipMalloc(&m->mgpoolb, tot * (int64_t)sizeof(double)));
   AGX_HIP(hipMemsetAsync(m->mgpoolb, 0, tot * sizeof(double), m->stream));
@@ -1540,6 +1898,8 @@ static int mp_create(agx_mesh *m) {
     B.u = p; p += n;
     B.src = p; p += n;
     B.uold = p; p += n;
+    B.tmp = p; p += n;
+    if (l < L - 1) { B.rhs = p; p += n; }
     B.bcv = p; p += pad32(3 * bghosts(B));
   }
   AGX_HIP(hipMalloc(&m->mpdev, sizeof(double) * (28 + NMOM * NPART)));
@@ -1674,6 +2034,68 @@ static void coarse_b32(agx_mesh *m, int top, int ni) {
   timer_end(m);
 }
 
+// Levels that run as whole passes (k_mg_down, k_mg_up): those above the coarse kernel's.  Every
+// extent above level 0 is even; a ring of four cells needs four to wrap once.
+template <typename LV>
+static bool pass_level(const LV &L) {
+  return std::min(L.n1, std::min(L.n2, L.n3)) >= 4;
+}
+// Planes per workgroup: a chunk runs about six iterations more than it has planes, so the
+// chunks are as long as 512 resident workgroups (two a CU) leave them.
+template <typename LV>
+static int pass_planes(const LV &L) {
+  const int64_t tiles = (int64_t)((L.n1 + TP_I - 1) / TP_I) * ((L.n2 + TP_J - 1) / TP_J);
+  int best = 2;
+  int64_t least = INT64_MAX;
+  for (int kc = 2; kc <= L.n3; kc += 2) {
+    const int64_t t = (kc + 6) * ((tiles * ((L.n3 + kc - 1) / kc) + 511) / 512);
+    if (t < least) { least = t; best = kc; }
+  }
+  return best;
+}
+template <typename T, typename LV>
+static PassArgs<T> pass_args(const agx_mesh *m, const LV &L) {
+  PassArgs<T> a = {};
+  a.n1 = L.n1; a.n2 = L.n2; a.n3 = L.n3;
+  a.kc = pass_planes(L);
+  a.dx2 = T(L.dx * L.dx);
+  a.idx2 = T(1.0 / (L.dx * L.dx));
+  a.isix = T(1.15 / 6.0);
+  a.c0 = m->coffset;
+  a.src = L.src;
+  return a;
+}
+template <typename T>
+static dim3 pass_grid(const PassArgs<T> &a) {
+  return dim3((unsigned)((a.n1 + TP_I - 1) / TP_I) * ((a.n2 + TP_J - 1) / TP_J) * ((a.n3 + a.kc - 1) / a.kc));
+}
+// framed level F of the multipole hierarchies (KIND BC_MP with FP64, BC_HOM with FP32);
+// bcv is null for BC_HOM
+template <typename T, int KIND, typename LV>
+static void down_b(agx_mesh *m, LV &F, LV &C, const double *bcv, bool fas) {
+  constexpr int NT = PassColumn<KIND, 2, 3, T>::NT;
+  PassArgs<T> a = pass_args<T>(m, F);
+  a.uin = F.u; a.uout = F.tmp;
+  a.rhs = F.rhs; a.old = F.uold;
+  a.csrc = C.src; a.cu = C.u;
+  a.bcv = bcv;
+  timer_begin(m, AGX_K_MG_SMOOTH);
+  if (fas) hipLaunchKernelGGL((k_mg_down<T, KIND, true>), pass_grid(a), dim3(NT), 0, m->stream, m->gate, a);
+  else hipLaunchKernelGGL((k_mg_down<T, KIND, false>), pass_grid(a), dim3(NT), 0, m->stream, m->gate, a);
+  timer_end(m);
+}
+template <typename T, int KIND, typename LV>
+static void up_b(agx_mesh *m, LV &F, LV &C, const double *bcv, bool fas) {
+  PassArgs<T> a = pass_args<T>(m, F);
+  a.uin = F.tmp; a.uout = F.u;
+  if (fas) a.src = F.rhs;
+  a.cc = C.u; a.ccold = C.uold;
+  a.bcv = bcv;
+  timer_begin(m, AGX_K_MG_SMOOTH);
+  hipLaunchKernelGGL((k_mg_up<T, KIND>), pass_grid(a), dim3(PassColumn<KIND, 1, 2, T>::NT), 0, m->stream, m->gate, a);
+  timer_end(m);
+}
+
 // SolveVCycle(1,1) (multigrid_driver.cpp:684-693) with the FAS steps of
 // OneStepToCoarser / SolveCoarsestGrid / OneStepToFiner (:583-677, :778-819) and the
 // MeshBlock task lists (mg_task_list.cpp:258-262, 287-510).  Boundaries are filled before
@@ -1689,6 +2111,11 @@ static void vcycle_b(agx_mesh *m) {
     while (m->current > ct) {
       const int l = m->current;
       MGLevelB &F = m->levb[l], &C = m->levb[l - 1];
+      if (m->mg_coarse && pass_level(F)) {
+        down_b<double, BC_MP>(m, F, C, F.bcv, l < m->fmglevel);
+        m->current--;
+        continue;
+      }
       bc_b(m, l);
       if (l < m->fmglevel) fas_b(m, l);
       smooth_b(m, l, 0);
@@ -1706,6 +2133,11 @@ static void vcycle_b(agx_mesh *m) {
     while (m->current < start) {
       const int l = m->current + 1;
       MGLevelB &F = m->levb[l], &C = m->levb[l - 1];
+      if (m->mg_coarse && pass_level(F)) {   // the coarse frame is filled: by k_mg_coarse or by k_mg_up
+        up_b<double, BC_MP>(m, F, C, F.bcv, l < m->fmglevel);
+        m->current++;
+        continue;
+      }
       bc_b(m, l - 1);
       timer_begin(m, AGX_K_MG_PROLONG);
       mb_prolong(m, C.u, C.uold, F.u, F.n1, F.n2, F.n3);
@@ -1817,6 +2249,11 @@ static void vcycle_b32(agx_mesh *m) {   // the per-level sequence of vcycle_b
   while (m->current > 0 && m->current > ct) {
     const int l = m->current;
     MGLevelB32 &F = m->levb32[l], &C = m->levb32[l - 1];
+    if (m->mg_coarse && pass_level(F)) {
+      down_b<float, BC_HOM>(m, F, C, nullptr, l < m->fmglevel);
+      m->current--;
+      continue;
+    }
     bc_b32(m, l);
     if (l < m->fmglevel) fas_b32(m, l);
     smooth_b32(m, l, 0);
@@ -1846,6 +2283,11 @@ static void vcycle_b32(agx_mesh *m) {   // the per-level sequence of vcycle_b
   while (m->current < start) {
     const int l = m->current + 1;
     MGLevelB32 &F = m->levb32[l], &C = m->levb32[l - 1];
+    if (m->mg_coarse && pass_level(F)) {
+      up_b<float, BC_HOM>(m, F, C, nullptr, l < m->fmglevel);
+      m->current++;
+      continue;
+    }
     bc_b32(m, l - 1);
     timer_begin(m, AGX_K_MG_PROLONG);
     mb_prolong(m, C.u, C.uold, F.u, F.n1, F.n2, F.n3);
@@ -2081,7 +2523,7 @@ int mg_create(agx_mesh *m) {
     if (m->mixed) {   // FP32 framed levels: correction, source, FAS copy
       m->levb32.resize(L);
       int64_t t32 = 0;
-      for (int l = 0; l < L; ++l) t32 += 3 * pad32(bcells(m->levb[l]));
+      for (int l = 0; l < L; ++l) t32 += (l < L - 1 ? 5 : 4) * pad32(bcells(m->levb[l]));
       AGX_HIP(hipMalloc(&m->mgpoolb32, t32 * (int64_t)sizeof(float)));
       AGX_HIP(hipMemsetAsync(m->mgpoolb32, 0, t32 * sizeof(float), m->stream));
       m->mg_bytes += t32 * (int64_t)sizeof(float);
@@ -2093,6 +2535,8 @@ int mg_create(agx_mesh *m) {
         B.u = q; q += n;
         B.src = q; q += n;
         B.uold = q; q += n;
+        B.tmp = q; q += n;
+        if (l < L - 1) { B.rhs = q; q += n; }
       }
     }
   }
@@ -2143,33 +2587,6 @@ static void smooth(agx_mesh *m, std::vector<MGLevelT<T>> &H, int l, int color) {
     hipLaunchKernelGGL(k_mg_smooth<T>, dim3(grid1d(n, BS)), dim3(BS), 0, m->stream, m->gate, L.u, L.src, L.n1, L.n2,
                        L.n3, T(dx2), T(isix), color ^ m->coffset);
   timer_end(m);
-}
-
-// One red-black pass (colour 0 then colour 1) on level l: fused into one launch into the
-// level's spare array (then swapped with u), or two sweeps.  By default the fused form
-// runs on FP64 levels of at least 2^26 cells.  Measured on MI355X (V(1,1) cycles/s, two
-// sweeps -> fused): 512^3 FP64 186 -> 231; at 256^3 (134 MB per level array, which the
-// 256 MB last-level cache holds between the two sweeps) two sweeps are faster (1746 vs
-// 1600), as they are for FP32 levels at 512^3 (231 vs 213).  agx_autotune times both
-// (mg_fuse 0 or 1: fused on every level of at least 2^21 cells) and keeps the faster;
-// the results are identical either way.
-template <typename T>
-static void smooth_pass(agx_mesh *m, std::vector<MGLevelT<T>> &H, int l) {
-  MGLevelT<T> &L = H[l];
-  const bool big = m->mg_fuse < 0 ? (sizeof(T) == 8 && lcells(L) >= ((int64_t)1 << 26))
-                                  : (m->mg_fuse == 1 && lcells(L) >= ((int64_t)1 << 21));
-  const bool fused = big && L.def && L.n1 % RB_TI == 0 && L.n2 % RB_TJ == 0 && (L.n3 & 1) == 0 && L.n3 >= 4;
-  if (!fused) {
-    smooth(m, H, l, 0);
-    smooth(m, H, l, 1);
-    return;
-  }
-  const int64_t nwg = (int64_t)(L.n1 / RB_TI) * (L.n2 / RB_TJ) * ((L.n3 + RB_KC - 1) / RB_KC);
-  timer_begin(m, AGX_K_MG_SMOOTH);
-  hipLaunchKernelGGL(k_mg_smooth_rb<T>, dim3((unsigned)nwg), dim3(RB_TI * RB_TJ), 0, m->stream, m->gate, L.u, L.def,
-                     L.src, L.n1, L.n2, L.n3, T(L.dx * L.dx), T(1.15 / 6.0), m->coffset);
-  timer_end(m);
-  std::swap(L.u, L.def);
 }
 
 template <typename T>
@@ -2304,24 +2721,58 @@ static void coarse_cycle(agx_mesh *m, std::vector<MGLevelT<T>> &H, int top, bool
   timer_end(m);
 }
 
+// A periodic level as whole passes; its spare array holds u between the way down and the way up.
+template <typename T>
+static void down_p(agx_mesh *m, MGLevelT<T> &F, MGLevelT<T> &C, bool first_sweep_done) {
+  PassArgs<T> a = pass_args<T>(m, F);
+  a.uin = F.u; a.uout = F.def;
+  a.csrc = C.src; a.cu = C.u;
+  a.first_sweep_done = first_sweep_done ? 1 : 0;
+  timer_begin(m, AGX_K_MG_SMOOTH);
+  hipLaunchKernelGGL((k_mg_down<T, BC_PER, false>), pass_grid(a), dim3(PassColumn<BC_PER, 2, 3, T>::NT), 0, m->stream,
+                     m->gate, a);
+  timer_end(m);
+}
+template <typename T>
+static void up_p(agx_mesh *m, MGLevelT<T> &F, MGLevelT<T> &C) {
+  PassArgs<T> a = pass_args<T>(m, F);
+  a.uin = F.def; a.uout = F.u;
+  a.cc = C.u;
+  timer_begin(m, AGX_K_MG_SMOOTH);
+  hipLaunchKernelGGL((k_mg_up<T, BC_PER>), pass_grid(a), dim3(PassColumn<BC_PER, 1, 2, T>::NT), 0, m->stream, m->gate,
+                     a);
+  timer_end(m);
+}
+
 template <typename T>
 static void vcycle(agx_mesh *m, std::vector<MGLevelT<T>> &H, bool first_sweep_done = false) {
   int start = m->current;
   m->coffset ^= 1;
   const int ct = coarse_top(H);
+  const bool passes = m->mg_fuse != 0;
   while (m->current > 0 && m->current > ct) {
     int l = m->current;
-    if (first_sweep_done && l == start) smooth(m, H, l, 1);
-    else smooth_pass(m, H, l);
-    defect_restrict(m, H, l);
+    const bool done = first_sweep_done && l == start;
+    if (passes && pass_level(H[l])) {
+      down_p(m, H[l], H[l - 1], done);
+    } else {
+      if (!done) smooth(m, H, l, 0);
+      smooth(m, H, l, 1);
+      defect_restrict(m, H, l);
+    }
     m->current--;
   }
   if (ct >= 0) coarse_cycle(m, H, m->current, first_sweep_done && m->current == start);
   else solve_coarsest(m, H);
   while (m->current < start) {
     int l = m->current + 1;
-    prolong(m, H, l);
-    smooth_pass(m, H, l);
+    if (passes && pass_level(H[l])) {
+      up_p(m, H[l], H[l - 1]);
+    } else {
+      prolong(m, H, l);
+      smooth(m, H, l, 0);
+      smooth(m, H, l, 1);
+    }
     m->current++;
   }
 }
@@ -2628,7 +3079,7 @@ int mg_solve_tail(agx_mesh *m) {
 }
 
 // Times V-cycles (on whatever the finest level holds; the next solve reloads it) with
-// the two red-black pass forms and keeps the faster (smooth_pass).
+// the levels as whole passes and as one launch per step, and keeps the faster.
 int mg_autotune(agx_mesh *m) {
   if (!m->mg_on || m->mp_on) return 0;
   hipEvent_t e0, e1;

@@ -335,18 +335,19 @@ int agx_mg_levels(agx_mesh *m, int32_t *nlevels, int32_t *dims, int32_t cap);
  * 512-thread workgroup; forms 4..5: the whole stage (fluxes in LDS) in one launch over
  * 16x16 or 32x8 columns.  Without autotuning each stage runs form 5, or on small meshes and
  * for PPM a split form.  With multigrid
- * gravity (periodic boundaries) it also times V-cycles with the red-black pass fused into
- * one launch and as two sweeps, and keeps the faster.  It writes only scratch registers
+ * gravity (periodic boundaries) it also times V-cycles with whole passes of a level (both
+ * sweeps and the transfer in one launch) and with one launch per step, and keeps the faster.  It writes only scratch registers
  * (u1, b1, fluxes, the multigrid levels, which every solve reloads), so call it between
  * cycles, e.g. after agx_initialize.  agx_set_tile forces a shape.  Results do not depend
  * on either choice. */
 int agx_autotune(agx_mesh *m, int32_t *choice);
 int agx_set_tile(agx_mesh *m, int32_t tile);   /* the same form for both stages */
-/* multigrid red-black pass form: -1 by level size (fused on FP64 levels of >= 2^26
- * cells, the default), 0 two sweeps, 1 fused on every level of >= 2^21 cells */
+/* Periodic V-cycles: levels above the coarse ones as whole passes, one launch down and one up
+ * (-1, the default, and 1), or one launch per step (0); identical potentials. */
 int agx_set_mg_fuse(agx_mesh *m, int32_t mode);
-/* Multipole V-cycles: run the coarse levels (at most 512 cells each) as one
- * single-workgroup launch (on = 1, the default) or one launch per step (0).  The
+/* Multipole V-cycles: run the coarse levels (at most 4096 cells each) as one
+ * single-workgroup launch and the others as whole passes, one launch down and one up (on = 1,
+ * the default), or one launch per step (0).  The
  * potentials are identical bit for bit; no counterpart in the reference.  Applies to
  * the FP64 V-cycles and to the FP32 correction cycles of the mixed form. */
 int agx_set_mg_coarse(agx_mesh *m, int32_t on);

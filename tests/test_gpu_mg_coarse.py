@@ -1,6 +1,7 @@
-"""k_mg_coarse against the per-level steps at the edges of its range: the whole hierarchy in the
-kernel (16^3 cells, and one 8^3 block), the largest level it takes, root grids that are odd or
-flat, and levels just above it; the same potential bit for bit."""
+"""k_mg_coarse, k_mg_down and k_mg_up against the per-level steps at the edges of their ranges: the
+whole hierarchy in the coarse kernel (16^3 cells, and one 8^3 block), root grids that are odd or
+flat, levels just above it, levels of one tile, of several and of parts of one, flat ones, and
+chunks that end inside; the same potential bit for bit."""
 import numpy as np
 import pytest
 
@@ -9,7 +10,8 @@ from tests.test_gpu_mg_levels import vcycle_by_steps
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [((8, 8, 8), 8), ((16, 16, 16), 8), ((24, 8, 8), 8), ((12, 20, 4), 4), ((64, 8, 4), 4), ((32, 32, 32), 8)]
+SHAPES = [((8, 8, 8), 8), ((16, 16, 16), 8), ((24, 8, 8), 8), ((12, 20, 4), 4), ((64, 8, 4), 4), ((32, 32, 32), 8),
+          ((40, 24, 56), 8), ((72, 16, 8), 8), ((96, 48, 16), 16), ((128, 128, 4), 4)]
 
 
 @pytest.mark.parametrize("precision", [0, 1])
@@ -54,3 +56,25 @@ def test_periodic_vcycle_identical(agx, n, b):
     assert np.array_equal(a.get("phi"), c.get("phi"))
     a.close()
     c.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("n,b", [((40, 24, 56), 8), ((64, 64, 64), 32), ((128, 32, 32), 32), ((128, 128, 4), 4),
+                                 ((96, 48, 16), 16), ((36, 20, 12), 4)])
+def test_periodic_passes_identical(agx, n, b, precision):
+    """whole passes against one launch per step"""
+    h = 1.0 / max(n)
+    d = make_desc(nx=n, bnx=(b, b, b), box=tuple((0.0, h * q) for q in n), self_gravity=1, mg_bc=0, mg_mode=0,
+                  four_pi_G=1.0, mg_threshold=-1.0, mg_niter=2, precision=precision)
+    U = np.zeros((5, n[2], n[1], n[0]))
+    U[0] = np.random.default_rng(5).uniform(0.5, 1.5, n[::-1])
+    ub = agx.scatter_cells(d, U)
+    out = []
+    for mode in (1, 0):
+        m = agx.Mesh(d)
+        m.set("u", ub)
+        m.set_mg_fuse(mode)
+        m.mg_solve(0)
+        out.append((m.get("phi"), m.mg_last()))
+        m.close()
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
