@@ -1312,90 +1312,99 @@ constexpr bool flux_flagged() {
   return std::is_same<T, float>::value && (ORDER == 3 || ORDER == ORDER_PPM_CHAR);
 }
 
-// One face of Hydro::CalculateFluxes in direction DIR: face_flux at (b, id), written to
+template <typename T>
+struct FluxArgs {
+  const T *w, *bcc;
+  const double *bn[3];                     // face field normal to each direction's faces
+  T *flx[3], *ey[3], *ez[3], *wct[3];
+  const BlockCoef *coef;
+  const double *plm;
+  const double *dtp;                       // device time step
+  double gamma, cs, dfl, pfl;
+  uint8_t *nearf;                          // near-tie flags of FP32 PPM, nflag bytes per direction
+  int64_t nflag;
+  int dir0, ndir;                          // the launch's directions
+};
+template <typename P>
+__device__ __forceinline__ P of_dir(P const (&p)[3], int dir) { return dir == 0 ? p[0] : (dir == 1 ? p[1] : p[2]); }
+
+// One face of Hydro::CalculateFluxes in direction dir: face_flux at (b, id), written to
 // the face arrays; FLAG also writes the face's near-tie flag (0 or 1) to nearf.
-template <int DIR, int ORDER, int RS, typename T, bool ISO, bool FLAG>
-__device__ __forceinline__ void flux_face(const Geo &g, int b, int64_t id, int cidx, const T *__restrict__ w,
-                                          const T *__restrict__ bcc, const double *__restrict__ bn,
-                                          T *__restrict__ flx, T *__restrict__ ey, T *__restrict__ ez,
-                                          T *__restrict__ wct, const BlockCoef *__restrict__ coef,
-                                          const double *__restrict__ plm, double gamma_, double cs_,
-                                          const double *__restrict__ dtp, double dfl_, double pfl_,
-                                          uint8_t *__restrict__ nearf) {
-  const int64_t sd[3] = {1, (int64_t)g.P, (int64_t)g.J * g.P};   // strides along i, j, k
-  const double *pc = plm + ((int64_t)b * 3 + DIR) * 2 * g.PL;    // [dxp][dxm] rows
+template <int ORDER, int RS, typename T, bool ISO, bool FLAG>
+__device__ __forceinline__ void flux_face(const Geo &g, const FluxArgs<T> &a, int dir, int b, int64_t id, int cidx) {
+  const int64_t sj = g.P, sk = (int64_t)g.J * g.P;   // strides along j, k
+  const int64_t st = dir == 0 ? 1 : (dir == 1 ? sj : sk), st1 = dir == 0 ? sj : (dir == 1 ? sk : 1),
+                st2 = dir == 0 ? sk : (dir == 1 ? 1 : sj);
+  const double *pc = a.plm + ((int64_t)b * 3 + dir) * 2 * g.PL;    // [dxp][dxm] rows
+  const int64_t fo = (int64_t)b * g.S + id;
   T f[5], fey, fez, fw;
   bool near;
-  face_flux<ORDER, RS, T, ISO, FLAG>(DIR, w + (int64_t)b * NHYDRO * g.S, bcc + (int64_t)b * 3 * g.S, g.S, id,
-                                     sd[DIR], sd[(DIR + 1) % 3], sd[(DIR + 2) % 3], pc, g.PL, cidx,
-                                     T(bn[(int64_t)b * g.S + id]), T(gamma_), T(cs_), T(dfl_), T(pfl_),
-                                     T(coef[b].dx[DIR]), T(*dtp), f, fey, fez, fw, &near);
-  constexpr int ivx = IVX + DIR, ivy = IVX + (DIR + 1) % 3, ivz = IVX + (DIR + 2) % 3;
-  T *fb = flx + (int64_t)b * NHYDRO * g.S + id;
+  face_flux<ORDER, RS, T, ISO, FLAG>(dir, a.w + (int64_t)b * NHYDRO * g.S, a.bcc + (int64_t)b * 3 * g.S, g.S, id, st,
+                                     st1, st2, pc, g.PL, cidx, T(of_dir(a.bn, dir)[fo]), T(a.gamma), T(a.cs),
+                                     T(a.dfl), T(a.pfl), T(a.coef[b].dx[dir]), T(*a.dtp), f, fey, fez, fw, &near);
+  const int ivx = IVX + dir, ivy = IVX + (dir == 2 ? 0 : dir + 1), ivz = IVX + (dir == 0 ? 2 : dir - 1);
+  T *fb = of_dir(a.flx, dir) + (int64_t)b * NHYDRO * g.S + id;
   fb[IDN * g.S] = f[0];
   fb[ivx * g.S] = f[1];
   fb[ivy * g.S] = f[2];
   fb[ivz * g.S] = f[3];
   if (!ISO) fb[IEN * g.S] = f[4];
-  int64_t fo = (int64_t)b * g.S + id;
-  ey[fo] = fey;
-  ez[fo] = fez;
-  wct[fo] = fw;
-  if constexpr (FLAG) nearf[fo] = near ? 1 : 0;
+  of_dir(a.ey, dir)[fo] = fey;
+  of_dir(a.ez, dir)[fo] = fez;
+  of_dir(a.wct, dir)[fo] = fw;
+  if constexpr (FLAG) a.nearf[dir * a.nflag + fo] = near ? 1 : 0;
 }
 
-// Hydro::CalculateFluxes for direction DIR, one thread per face (face_flux).  For FP32 PPM
-// nearf (one byte per cell of the block arrays) receives each face's near-tie flag.
-template <int DIR, int ORDER, int RS, typename T, bool ISO>
+// Hydro::CalculateFluxes, one thread per face (face_flux), the directions of the launch in one
+// grid: a workgroup's direction is blockIdx.x mod ndir (in the XCD-aware order), so the three
+// directions of a piece of a plane run together and share its lines of w and bcc, and a small
+// mesh fills the chip once instead of three times.  Cycles in us, three launches against one
+// (with the time step's two launches made one, 4 us): 64 x 32 x 32 FP64 PLM 119 : 95, 64^3
+// 246 : 215, 120 x 90 x 70 PPM 913 : 883, 256^3 mixed 6797 : 6556.  Bound by FP64 and reciprocal
+// issue on large meshes.  For FP32 PPM nearf (one byte per cell of the block arrays and
+// direction) receives each face's near-tie flag.
+template <int ORDER, int RS, typename T, bool ISO>
 __global__ void __launch_bounds__(256)
-k_flux(Geo g, const T *__restrict__ w, const T *__restrict__ bcc,
-       const double *__restrict__ bn, T *__restrict__ flx, T *__restrict__ ey,
-       T *__restrict__ ez, T *__restrict__ wct, const BlockCoef *__restrict__ coef,
-       const double *__restrict__ plm, double gamma_, double cs_, const double *__restrict__ dtp, double dfl_,
-       double pfl_, uint8_t *__restrict__ nearf) {
-  int il = g.is - (DIR != 0), iu = g.ie + 1;
-  int jl = g.js - (DIR != 1), ju = g.je + 1;
-  int kl = g.ks - (DIR != 2);
-  PlaneIdx p;
-  if (!plane_index(il, iu, jl, ju, kl, p, DIR == 2)) return;   // x3: 4-plane stencil
-  const int cidx = (DIR == 0) ? p.i : (DIR == 1 ? p.j : p.k);   // index of the cell above the face
-  flux_face<DIR, ORDER, RS, T, ISO, flux_flagged<ORDER, T>()>(g, p.b, IDX(g, p.k, p.j, p.i), cidx, w, bcc, bn,
-                                                                flx, ey, ez, wct, coef, plm, gamma_, cs_, dtp,
-                                                                dfl_, pfl_, nearf);
+k_flux(Geo g, FluxArgs<T> a) {
+  const uint3 wg = xcd_block();
+  const int part = (int)(wg.x / (unsigned)a.ndir), dir = a.dir0 + (int)(wg.x - part * (unsigned)a.ndir);
+  const int il = g.is - (dir != 0), jl = g.js - (dir != 1), k = g.ks - (dir != 2) + (int)wg.y, b = wg.z;
+  const unsigned ni = g.ie + 1 - il + 1, nj = g.je + 1 - jl + 1, q = part * 256u + threadIdx.x;
+  if (q >= ni * nj || k > g.ke + 1) return;
+  const unsigned qj = q / ni;
+  const int j = jl + (int)qj, i = il + (int)(q - qj * ni);
+  const int cidx = dir == 0 ? i : (dir == 1 ? j : k);   // index of the cell above the face
+  flux_face<ORDER, RS, T, ISO, flux_flagged<ORDER, T>()>(g, a, dir, b, IDX(g, k, j, i), cidx);
 }
 
 // Second pass of FP32 PPM fluxes: each workgroup scans FIX_SPAN bytes of nearf (16 per
 // thread, one 16-byte load), gathers the flagged faces into an LDS list, clears their
 // flags (so nearf is all zero between passes) and recomputes those faces with the FP64
 // re-run of the limiter, so the near-tie faces occupy whole waves instead of single
-// lanes of every wave of k_flux.  nflag (the length of nearf) is a multiple of FIX_SPAN.
+// lanes of every wave of k_flux.  nflag (the flags of one direction) is a multiple of FIX_SPAN.
 constexpr int FIX_PER = 16, FIX_SPAN = 256 * FIX_PER;
-template <int DIR, int ORDER, int RS, bool ISO>
+template <int ORDER, int RS, bool ISO>
 __global__ void __launch_bounds__(256)
-k_flux_fix(Geo g, const float *__restrict__ w, const float *__restrict__ bcc,
-           const double *__restrict__ bn, float *__restrict__ flx, float *__restrict__ ey,
-           float *__restrict__ ez, float *__restrict__ wct, const BlockCoef *__restrict__ coef,
-           const double *__restrict__ plm, double gamma_, double cs_, const double *__restrict__ dtp,
-           double dfl_, double pfl_, uint8_t *__restrict__ nearf, int64_t nflag) {
+k_flux_fix(Geo g, FluxArgs<float> a) {
   __shared__ int list[FIX_SPAN];
   __shared__ int cnt;
   if (threadIdx.x == 0) cnt = 0;
   __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * FIX_SPAN;
-  const int64_t off = base + (int64_t)threadIdx.x * FIX_PER;
-  if (off < nflag) {
-    uint4 v = *reinterpret_cast<const uint4 *>(nearf + off);
-    if (v.x | v.y | v.z | v.w) {
-      const uint32_t wv[4] = {v.x, v.y, v.z, v.w};
+  const unsigned spans = (unsigned)(a.nflag / FIX_SPAN);
+  const int dir = a.dir0 + (int)(blockIdx.x / spans);
+  const int64_t base = (int64_t)(blockIdx.x % spans) * FIX_SPAN;
+  uint8_t *flags = a.nearf + dir * a.nflag + base + (int64_t)threadIdx.x * FIX_PER;
+  uint4 v = *reinterpret_cast<const uint4 *>(flags);
+  if (v.x | v.y | v.z | v.w) {
+    const uint32_t wv[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-      for (int t = 0; t < FIX_PER; ++t)
-        if ((wv[t >> 2] >> (8 * (t & 3))) & 0xffu) list[atomicAdd(&cnt, 1)] = threadIdx.x * FIX_PER + t;
-      *reinterpret_cast<uint4 *>(nearf + off) = make_uint4(0u, 0u, 0u, 0u);
-    }
+    for (int t = 0; t < FIX_PER; ++t)
+      if ((wv[t >> 2] >> (8 * (t & 3))) & 0xffu) list[atomicAdd(&cnt, 1)] = threadIdx.x * FIX_PER + t;
+    *reinterpret_cast<uint4 *>(flags) = make_uint4(0u, 0u, 0u, 0u);
   }
   __syncthreads();
   const int n = cnt;
-  const int il = g.is - (DIR != 0), jl = g.js - (DIR != 1), kl = g.ks - (DIR != 2);
+  const int il = g.is - (dir != 0), jl = g.js - (dir != 1), kl = g.ks - (dir != 2);
   for (int e = threadIdx.x; e < n; e += 256) {
     const int64_t fo = base + list[e];
     const int b = (int)(fo / g.S);
@@ -1405,9 +1414,8 @@ k_flux_fix(Geo g, const float *__restrict__ w, const float *__restrict__ bcc,
     const int j = r / g.P, i = r - j * g.P;
     // only faces of this direction are ever flagged; the test keeps the stencil in range
     if (b >= g.nb || i < il || i > g.ie + 1 || j < jl || j > g.je + 1 || k < kl || k > g.ke + 1) continue;
-    const int cidx = (DIR == 0) ? i : (DIR == 1 ? j : k);
-    flux_face<DIR, ORDER, RS, float, ISO, false>(g, b, id, cidx, w, bcc, bn, flx, ey, ez, wct, coef, plm, gamma_,
-                                                 cs_, dtp, dfl_, pfl_, nullptr);
+    const int cidx = dir == 0 ? i : (dir == 1 ? j : k);
+    flux_face<ORDER, RS, float, ISO, false>(g, a, dir, b, id, cidx);
   }
 }
 
@@ -2777,8 +2785,8 @@ int agx_mesh_create(const agx_mesh_desc *desc, agx_mesh **out) {
   if (e == hipSuccess) e = hipMalloc(&m->cellvol, sizeof(double) * g.nb);
   if (m->mixed && g.ng >= 3) {   // near-tie flags of the FP32 PPM flux pass, all zero between passes
     m->nearf_n = ((int64_t)g.nb * g.S + FIX_SPAN - 1) / FIX_SPAN * FIX_SPAN;
-    if (e == hipSuccess) e = hipMalloc(&m->nearf, m->nearf_n);
-    if (e == hipSuccess) e = hipMemsetAsync(m->nearf, 0, m->nearf_n, m->stream);
+    if (e == hipSuccess) e = hipMalloc(&m->nearf, 3 * m->nearf_n);
+    if (e == hipSuccess) e = hipMemsetAsync(m->nearf, 0, 3 * m->nearf_n, m->stream);
   }
   // Coordinates::CellVolume, Cartesian: dx1f*dx2f*dx3f (coordinates.cpp:521-531)
   std::vector<double> vol_h(g.nb);
@@ -3133,17 +3141,23 @@ __global__ void k_set_scalars(double *__restrict__ s, double dt, double time, do
   }
 }
 
-// End of a cycle on the device: time += dt, then Mesh::NewTimeStep (mesh.cpp:1078-1119)
-// from the block minimum in s[0] (k_min_final): dt = min(cfl * min, 2 dt), clipped to
-// tlim - time.  The same operations as agx_cycle's host path.
-__global__ void k_advance(double *__restrict__ s, double cfl) {
+// End of a cycle on the device: the least of the n time-step partials, time += dt, then
+// Mesh::NewTimeStep (mesh.cpp:1078-1119): dt = min(cfl * min, 2 dt), clipped to tlim - time.
+// The same operations as agx_cycle's host path.
+__global__ void __launch_bounds__(256) k_advance(const double *__restrict__ part, int64_t n, double *__restrict__ s,
+                                                 double cfl) {
+  __shared__ double sh[4];
+  const double dt = s[SC_DT], tlim = s[SC_TLIM], time = s[SC_TIME] + dt;
+  double m = DBL_MAX;
+#pragma unroll 4
+  for (int64_t q = threadIdx.x; q < n; q += 256) m = dmin(m, part[q]);
+  m = wg_min256(m, sh);
   if (threadIdx.x == 0) {
-    const double dt = s[SC_DT], tlim = s[SC_TLIM];
-    const double time = s[SC_TIME] + dt;
-    const double bdt = s[0] * cfl;
+    const double bdt = m * cfl;
     double ndt = 2.0 * dt;
     ndt = (bdt < ndt) ? bdt : ndt;
     if (time < tlim && (tlim - time) < ndt) ndt = tlim - time;
+    s[0] = m;
     s[SC_TIME] = time;
     s[SC_DT] = ndt;
   }
@@ -3220,72 +3234,74 @@ int agx_calculate_fluxes(agx_mesh *m, int order) {
 }
 
 extern "C++" {
-// k_flux in direction DIR from the face-centred field B to the face arrays F, EY, EZ, WX;
-// FP32 PPM adds the k_flux_fix pass over the faces k_flux flagged.
-template <int DIR, int ORD, int RS, typename TW, bool ISO>
-static void launch_flux(agx_mesh *m, int B, int F, int EY, int EZ, int WX) {
+// k_flux in the directions dir0 .. dir0 + ndir - 1; FP32 PPM adds the k_flux_fix pass over the
+// faces k_flux flagged
+template <int ORD, int RS, typename TW, bool ISO>
+static void launch_flux(agx_mesh *m, int dir0, int ndir) {
   const Geo &g = m->g;
   double **A = m->arr.a;
-  hipLaunchKernelGGL((k_flux<DIR, ORD, RS, TW, ISO>),
-                     plane_grid(g.is - (DIR != 0), g.ie + 1, g.js - (DIR != 1), g.je + 1, g.ks - (DIR != 2),
-                                g.ke + 1, g.nb),
-                     dim3(256), 0, m->stream, g, as<TW>(A[AGX_ARR_W]), as<TW>(A[AGX_ARR_BCC]), A[B], as<TW>(A[F]),
-                     as<TW>(A[EY]), as<TW>(A[EZ]), as<TW>(A[WX]), m->coef, m->plm, m->d.gamma, m->d.iso_cs,
-                     m->scal + SC_DT, m->d.dfloor, m->d.pfloor, m->nearf);
-  if constexpr (flux_flagged<ORD, TW>()) {
-    hipLaunchKernelGGL((k_flux_fix<DIR, ORD, RS, ISO>), dim3((unsigned)(m->nearf_n / FIX_SPAN)), dim3(256), 0,
-                       m->stream, g, as<float>(A[AGX_ARR_W]), as<float>(A[AGX_ARR_BCC]), A[B], as<float>(A[F]),
-                       as<float>(A[EY]), as<float>(A[EZ]), as<float>(A[WX]), m->coef, m->plm, m->d.gamma,
-                       m->d.iso_cs, m->scal + SC_DT, m->d.dfloor, m->d.pfloor, m->nearf, m->nearf_n);
+  FluxArgs<TW> a;
+  a.w = as<TW>(A[AGX_ARR_W]); a.bcc = as<TW>(A[AGX_ARR_BCC]);
+  // face EMF targets: x1 -> (e3_x1f, e2_x1f), x2 -> (e1_x2f, e3_x2f), x3 -> (e2_x3f, e1_x3f)
+  // (calculate_fluxes.cpp:86,200,306)
+  static const int arr[3][5] = {{AGX_ARR_B1F, AGX_ARR_FX1, AGX_ARR_E3X1, AGX_ARR_E2X1, AGX_ARR_WX1},
+                                {AGX_ARR_B2F, AGX_ARR_FX2, AGX_ARR_E1X2, AGX_ARR_E3X2, AGX_ARR_WX2},
+                                {AGX_ARR_B3F, AGX_ARR_FX3, AGX_ARR_E2X3, AGX_ARR_E1X3, AGX_ARR_WX3}};
+  for (int d = 0; d < 3; ++d) {
+    a.bn[d] = A[arr[d][0]];
+    a.flx[d] = as<TW>(A[arr[d][1]]);
+    a.ey[d] = as<TW>(A[arr[d][2]]);
+    a.ez[d] = as<TW>(A[arr[d][3]]);
+    a.wct[d] = as<TW>(A[arr[d][4]]);
   }
+  a.coef = m->coef;
+  a.plm = m->plm;
+  a.dtp = m->scal + SC_DT;
+  a.gamma = m->d.gamma; a.cs = m->d.iso_cs; a.dfl = m->d.dfloor; a.pfl = m->d.pfloor;
+  a.nearf = m->nearf; a.nflag = m->nearf_n;
+  a.dir0 = dir0; a.ndir = ndir;
+  // the largest plane of faces (x3: two more cells each way) and the most planes (x1, x2)
+  const dim3 grid(ndir * grid1d((int64_t)(g.bx1 + 2) * (g.bx2 + 2), 256), (unsigned)(g.bx3 + 2), (unsigned)g.nb);
+  hipLaunchKernelGGL((k_flux<ORD, RS, TW, ISO>), grid, dim3(256), 0, m->stream, g, a);
+  if constexpr (flux_flagged<ORD, TW>())
+    hipLaunchKernelGGL((k_flux_fix<ORD, RS, ISO>), dim3(ndir * (unsigned)(m->nearf_n / FIX_SPAN)), dim3(256), 0,
+                       m->stream, g, a);
+}
+
+template <int ORD, int RS, bool ISO>
+static void launch_flux_prec(agx_mesh *m, int dir0, int ndir) {
+  if (m->mixed) launch_flux<ORD, RS, float, ISO>(m, dir0, ndir);
+  else launch_flux<ORD, RS, double, ISO>(m, dir0, ndir);
+}
+template <int ORD>
+static void launch_flux_order(agx_mesh *m, int dir0, int ndir) {
+  const int rs = m->d.rsolver;
+  if (rs == AGX_RSOLVER_LHLLD) launch_flux_prec<ORD, AGX_RSOLVER_LHLLD, false>(m, dir0, ndir);
+  else if (m->iso && rs == AGX_RSOLVER_HLLE) launch_flux_prec<ORD, AGX_RSOLVER_HLLE, true>(m, dir0, ndir);
+  else if (m->iso) launch_flux_prec<ORD, AGX_RSOLVER_HLLD, true>(m, dir0, ndir);
+  else if (rs == AGX_RSOLVER_HLLE) launch_flux_prec<ORD, AGX_RSOLVER_HLLE, false>(m, dir0, ndir);
+  else if (rs == AGX_RSOLVER_ROE) launch_flux_prec<ORD, AGX_RSOLVER_ROE, false>(m, dir0, ndir);
+  else launch_flux_prec<ORD, AGX_RSOLVER_HLLD, false>(m, dir0, ndir);
 }
 }  // extern "C++"
 
 static int calculate_fluxes(agx_mesh *m, int order) {
   if (order < 1 || order > 3) { set_error("order %d not supported", order); return -2; }
   if (order == 3 && m->g.ng < 3) { set_error("PPM needs nghost >= 3 (reconstruction.cpp:90-100)"); return -3; }
-  const int rs = m->d.rsolver;
-#define FLUX_LAUNCH_T(DIR, ORD, RS, B, F, EY, EZ, WX, TW, ISO)                                 \
-  launch_flux<DIR, ORD, RS, TW, ISO>(m, B, F, EY, EZ, WX)
-#define FLUX_LAUNCH_E(DIR, ORD, RS, B, F, EY, EZ, WX, ISO)                                     \
-  if (m->mixed) FLUX_LAUNCH_T(DIR, ORD, RS, B, F, EY, EZ, WX, float, ISO);                    \
-  else FLUX_LAUNCH_T(DIR, ORD, RS, B, F, EY, EZ, WX, double, ISO)
-#define FLUX_LAUNCH(DIR, ORD, RS, B, F, EY, EZ, WX)                                            \
-  if (m->iso) { FLUX_LAUNCH_E(DIR, ORD, (RS == AGX_RSOLVER_HLLE ? AGX_RSOLVER_HLLE : AGX_RSOLVER_HLLD), \
-                              B, F, EY, EZ, WX, true); }                                       \
-  else { FLUX_LAUNCH_E(DIR, ORD, RS, B, F, EY, EZ, WX, false); }
-#define FLUX_ORD(DIR, ORD, B, F, EY, EZ, WX)                                                    \
-  if (rs == AGX_RSOLVER_HLLE) { FLUX_LAUNCH(DIR, ORD, AGX_RSOLVER_HLLE, B, F, EY, EZ, WX); }    \
-  else if (rs == AGX_RSOLVER_ROE) { FLUX_LAUNCH(DIR, ORD, AGX_RSOLVER_ROE, B, F, EY, EZ, WX); } \
-  else if (rs == AGX_RSOLVER_LHLLD) { FLUX_LAUNCH_E(DIR, ORD, AGX_RSOLVER_LHLLD, B, F, EY, EZ, WX, false); } \
-  else { FLUX_LAUNCH(DIR, ORD, AGX_RSOLVER_HLLD, B, F, EY, EZ, WX); }
   // xorder "2c"/"3c": PLM/PPM limited in characteristic variables
   const bool chp = m->d.char_proj && order > 1;
-#define FLUX_DIR(DIR, B, F, EY, EZ, WX)                                                         \
-  timer_begin(m, AGX_K_FLUX_X1 + DIR);                                                        \
-  if (order == 1) {                                                                           \
-    FLUX_ORD(DIR, 1, B, F, EY, EZ, WX)                                                        \
-  } else if (order == 2 && chp) {                                                             \
-    FLUX_ORD(DIR, ORDER_PLM_CHAR, B, F, EY, EZ, WX)                                           \
-  } else if (order == 2) {                                                                    \
-    FLUX_ORD(DIR, 2, B, F, EY, EZ, WX)                                                        \
-  } else if (chp) {                                                                           \
-    FLUX_ORD(DIR, ORDER_PPM_CHAR, B, F, EY, EZ, WX)                                           \
-  } else {                                                                                    \
-    FLUX_ORD(DIR, 3, B, F, EY, EZ, WX)                                                        \
-  }                                                                                           \
-  timer_end(m);                                                                               \
-  LAUNCH_CHECK("k_flux");
-  // face EMF targets: x1 -> (e3_x1f, e2_x1f), x2 -> (e1_x2f, e3_x2f), x3 -> (e2_x3f, e1_x3f)
-  // (calculate_fluxes.cpp:86,200,306)
-  FLUX_DIR(0, AGX_ARR_B1F, AGX_ARR_FX1, AGX_ARR_E3X1, AGX_ARR_E2X1, AGX_ARR_WX1)
-  FLUX_DIR(1, AGX_ARR_B2F, AGX_ARR_FX2, AGX_ARR_E1X2, AGX_ARR_E3X2, AGX_ARR_WX2)
-  FLUX_DIR(2, AGX_ARR_B3F, AGX_ARR_FX3, AGX_ARR_E2X3, AGX_ARR_E1X3, AGX_ARR_WX3)
-#undef FLUX_DIR
-#undef FLUX_ORD
-#undef FLUX_LAUNCH
-#undef FLUX_LAUNCH_E
-#undef FLUX_LAUNCH_T
+  // one launch, or one per direction while each direction's time is being taken
+  const int ndir = m->timer.enabled ? 1 : 3;
+  for (int d = 0; d < 3; d += ndir) {
+    timer_begin(m, AGX_K_FLUX_X1 + d);
+    if (order == 1) launch_flux_order<1>(m, d, ndir);
+    else if (order == 2 && chp) launch_flux_order<ORDER_PLM_CHAR>(m, d, ndir);
+    else if (order == 2) launch_flux_order<2>(m, d, ndir);
+    else if (chp) launch_flux_order<ORDER_PPM_CHAR>(m, d, ndir);
+    else launch_flux_order<3>(m, d, ndir);
+    timer_end(m);
+    LAUNCH_CHECK("k_flux");
+  }
   return 0;
 }
 
@@ -3691,8 +3707,8 @@ static int cycle_device(agx_mesh *m) {
   if (!rc) rc = stage_fused(m, 2, true);
   if (!rc && m->d.self_gravity) rc = mg_solve(m, 2);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_min_final, dim3(1), dim3(256), 0, m->stream, m->dtpart, (int64_t)sg.x * sg.y * sg.z, m->scal);
-  hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, m->stream, m->scal, m->d.cfl);
+  hipLaunchKernelGGL(k_advance, dim3(1), dim3(256), 0, m->stream, m->dtpart, (int64_t)sg.x * sg.y * sg.z, m->scal,
+                     m->d.cfl);
   LAUNCH_CHECK("k_advance");
   return 0;
 }
@@ -3783,8 +3799,8 @@ static int cycle_segment(agx_mesh *m, int seg, int k, std::vector<MGSnap> &snaps
     return 0;
   }
   const dim3 sg = stage_grid(m->g, m->tile);
-  hipLaunchKernelGGL(k_min_final, dim3(1), dim3(256), 0, m->stream, m->dtpart, (int64_t)sg.x * sg.y * sg.z, m->scal);
-  hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, m->stream, m->scal, m->d.cfl);
+  hipLaunchKernelGGL(k_advance, dim3(1), dim3(256), 0, m->stream, m->dtpart, (int64_t)sg.x * sg.y * sg.z, m->scal,
+                     m->d.cfl);
   LAUNCH_CHECK("k_advance");
   snaps.assign(1, mg_snap(m));
   return 0;
