@@ -369,10 +369,8 @@ k_mg_partial(const int *__restrict__ gate, const T *__restrict__ a, const T *__r
   if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
-__global__ void __launch_bounds__(BS) k_mg_final(const int *__restrict__ gate,
-                                  const double *__restrict__ part, int64_t n,
-                                                 double *__restrict__ out) {
-  if (gate && *gate) return;   // a closed gate: the recorded V-cycle loop has ended
+// the sum of n partials, in thread 0 (fixed order)
+__device__ __forceinline__ double part_sum(const double *__restrict__ part, int64_t n) {
   __shared__ double sh[BS];
   double v = 0.0;
 #pragma unroll 8
@@ -383,7 +381,46 @@ __global__ void __launch_bounds__(BS) k_mg_final(const int *__restrict__ gate,
     if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
     __syncthreads();
   }
-  if (threadIdx.x == 0) *out = sh[0];
+  return sh[0];
+}
+
+__global__ void __launch_bounds__(BS) k_mg_final(const int *__restrict__ gate, const double *__restrict__ part,
+                                                 int64_t n, double *__restrict__ out) {
+  if (gate && *gate) return;   // a closed gate: the recorded V-cycle loop has ended
+  const double sum = part_sum(part, n);
+  if (threadIdx.x == 0) *out = sum;
+}
+
+// finish_norm on the device: sqrt(sum * dv / volume)
+__global__ void k_mg_gate_open(MGGate *g, const double *__restrict__ scal, double dv, double vol, double eps) {
+  if (threadIdx.x) return;
+  const double def = sqrt(scal[0] * dv / vol);
+  g->iters = 0;
+  g->def = def;
+  g->closed = (def > eps) ? 0 : 1;
+}
+
+// SolveIterative's tests after a V-cycle (multigrid_driver.cpp:733-753); n is the
+// loop's count before its increment
+__device__ __forceinline__ void gate_check(MGGate *g, double sum, double dv, double vol, double eps) {
+  const double olddef = g->def;
+  const double def = sqrt(sum * dv / vol);
+  const int n = g->iters;
+  g->iters = n + 1;
+  g->def = def;
+  if ((def / olddef > 0.8 && eps == 0.0) || n > 100 || !(def > eps)) g->closed = 1;
+}
+
+// k_mg_final for the norm that ends a pass of the recorded loop, and the gate's check of it:
+// one launch of 4.6 us where the two took 9
+__global__ void __launch_bounds__(BS) k_mg_final_check(const double *__restrict__ part, int64_t n,
+                                                       double *__restrict__ out, MGGate *g, double dv, double vol,
+                                                       double eps) {
+  const int closed = g->closed;
+  const double sum = part_sum(part, n);
+  if (closed || threadIdx.x) return;
+  *out = sum;
+  gate_check(g, sum, dv, vol, eps);
 }
 
 template <typename T>
@@ -1867,8 +1904,21 @@ static int64_t pad32(int64_t n) { return (n + 63) / 64 * 64; }   // 64 elements:
 static int64_t npart(int64_t n) { return std::min<int64_t>(grid1d(n, BS), NPART); }
 
 static double finish_norm(agx_mesh *m);
+static int iterate(agx_mesh *m, int &iters, double &def);
 static void first_defect_sum(agx_mesh *m);
 static void loop_step(agx_mesh *m);
+static double mesh_volume(const agx_mesh_desc &d);
+static double norm_dv(const agx_mesh *m) { return m->rdx_blk * m->rdy_blk * m->rdz_blk; }
+
+// the nb partials in red summed into scal[slot]; slot 0 is the defect norm, which ends a gated
+// pass and is checked there (k_mg_final_check)
+static void final_sum(agx_mesh *m, int64_t nb, int slot) {
+  if (m->gate && slot == 0)
+    hipLaunchKernelGGL(k_mg_final_check, dim3(1), dim3(BS), 0, m->stream, m->red, nb, m->scal, m->gatedev, norm_dv(m),
+                       mesh_volume(m->d), m->mg_eps);
+  else
+    hipLaunchKernelGGL(k_mg_final, dim3(1), dim3(BS), 0, m->stream, m->gate, m->red, nb, m->scal + slot);
+}
 
 // ---------------------------------------------------------------- multipole hierarchy
 static int64_t bcells(const MGLevelB &L) { return (int64_t)(L.n1 + 2) * (L.n2 + 2) * (L.n3 + 2); }
@@ -2332,7 +2382,7 @@ static void defect_sum_b(agx_mesh *m) {
   const int64_t nb = npart((int64_t)F.n1 * F.n2 * F.n3);
   hipLaunchKernelGGL(k_mb_defect_partial, dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, F.u, F.src, F.n1,
                      F.n2, F.n3, 1.0 / (F.dx * F.dx), m->red);
-  hipLaunchKernelGGL(k_mg_final, dim3(1), dim3(BS), 0, m->stream, m->gate, m->red, nb, m->scal);
+  final_sum(m, nb, 0);
 }
 static double defect_norm_b(agx_mesh *m) {
   defect_sum_b(m);
@@ -2405,21 +2455,10 @@ static int retrieve_b(agx_mesh *m) {
 static int mg_solve_b(agx_mesh *m, int stage) {
   solve_load_b(m);
   int iters = 0;
+  double def = 0.0;
   if (m->mg_eps >= 0.0) {   // SolveIterative, multigrid_driver.cpp:721-755
-    first_defect_sum(m);
-    double def = finish_norm(m);
-    int n = 0;
-    while (def > m->mg_eps) {
-      loop_step(m);   // correction_step_b (mixed) or vcycle_b, then defect_sum_b
-      iters++;
-      double olddef = def;
-      def = finish_norm(m);
-      if (def / olddef > 0.8) {
-        if (m->mg_eps == 0.0) break;
-      }
-      if (n > 100) break;
-      n++;
-    }
+    int rc = iterate(m, iters, def);
+    if (rc) return rc;
     m->last_norm = def;
     if (stage == 1 || stage == 2) m->mg_kpred[stage - 1] = iters;
   } else {   // SolveIterativeFixedTimes, multigrid_driver.cpp:762-771
@@ -2635,7 +2674,7 @@ static void level_sum(agx_mesh *m, std::vector<MGLevelT<T>> &H, int l, int mode,
   else
     hipLaunchKernelGGL((k_mg_partial<1, T>), dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, L.u, L.src, L.n1,
                        L.n2, L.n3, T(idx2), m->red);
-  hipLaunchKernelGGL(k_mg_final, dim3(1), dim3(BS), 0, m->stream, m->gate, m->red, nb, m->scal + slot);
+  final_sum(m, nb, slot);
   timer_end(m);
 }
 
@@ -2644,7 +2683,7 @@ static void level_sum_src(agx_mesh *m, int l, int slot) {
   int64_t nb = npart(lcells(L));
   hipLaunchKernelGGL((k_mg_partial<0, double>), dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, L.src, L.src,
                      L.n1, L.n2, L.n3, 0.0, m->red);
-  hipLaunchKernelGGL(k_mg_final, dim3(1), dim3(BS), 0, m->stream, m->gate, m->red, nb, m->scal + slot);
+  final_sum(m, nb, slot);
 }
 
 static double mesh_volume(const agx_mesh_desc &d) {
@@ -2841,7 +2880,7 @@ static void defect_to32(agx_mesh *m, bool correct) {
     hipLaunchKernelGGL(k_mg_defect_to32, dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, F.u,
                        correct ? F32.u : (const float *)nullptr, correct ? F.def : (double *)nullptr, F.src,
                        F32.src, F32.def, F.n1, F.n2, F.n3, idx2, dx2f, isixf, cred, m->red);
-  hipLaunchKernelGGL(k_mg_final, dim3(1), dim3(BS), 0, m->stream, m->gate, m->red, nb, m->scal);
+  final_sum(m, nb, 0);
   timer_end(m);
   if (correct) std::swap(F.u, F.def);
   std::swap(F32.u, F32.def);
@@ -2921,21 +2960,10 @@ int mg_solve(agx_mesh *m, int stage) {
   const bool mixed = m->mixed;
   solve_load(m);
   int iters = 0;
+  double def = 0.0;
   if (m->mg_eps >= 0.0) {   // SolveIterative, multigrid_driver.cpp:721-755
-    first_defect_sum(m);
-    double def = finish_norm(m);
-    int n = 0;
-    while (def > m->mg_eps) {
-      loop_step(m);
-      iters++;
-      double olddef = def;
-      def = finish_norm(m);
-      if (def / olddef > 0.8) {
-        if (m->mg_eps == 0.0) break;
-      }
-      if (n > 100) break;
-      n++;
-    }
+    int rc = iterate(m, iters, def);
+    if (rc) return rc;
     m->last_norm = def;
     if (stage == 1 || stage == 2) m->mg_kpred[stage - 1] = iters;
     subtract_average(m, 1);
@@ -2958,34 +2986,13 @@ int mg_solve(agx_mesh *m, int stage) {
 // ---- a threshold solve recorded into a graph
 //
 // The loop's V-cycle count is only known on the device, so the recorded loop runs k
-// passes whose kernels all take the gate: after each pass k_mg_gate_check applies the
+// passes whose kernels all take the gate: after each pass k_mg_final_check applies the
 // loop's stopping rule to the new norm, and once it closes the gate the remaining passes
 // return at once.  The host state a pass changes (red-black offset, swapped arrays) is
 // captured after every recorded pass; mg_solve_settle reads how many passes ran and
 // restores the state after that many, then runs any further passes eagerly as mg_solve
 // would.  Every pass that runs is the same kernel sequence as mg_solve's, so the result
 // is the eager one bit for bit.
-
-// finish_norm on the device: sqrt(sum * dv / volume)
-__global__ void k_mg_gate_open(MGGate *g, const double *__restrict__ scal, double dv, double vol, double eps) {
-  if (threadIdx.x) return;
-  const double def = sqrt(scal[0] * dv / vol);
-  g->iters = 0;
-  g->def = def;
-  g->closed = (def > eps) ? 0 : 1;
-}
-
-// SolveIterative's tests after a V-cycle (multigrid_driver.cpp:733-753); n is the
-// loop's count before its increment
-__global__ void k_mg_gate_check(MGGate *g, const double *__restrict__ scal, double dv, double vol, double eps) {
-  if (threadIdx.x || g->closed) return;
-  const double olddef = g->def;
-  const double def = sqrt(scal[0] * dv / vol);
-  const int n = g->iters;
-  g->iters = n + 1;
-  g->def = def;
-  if ((def / olddef > 0.8 && eps == 0.0) || n > 100 || !(def > eps)) g->closed = 1;
-}
 
 MGSnap mg_snap(const agx_mesh *m) {
   MGSnap s;
@@ -3015,8 +3022,6 @@ std::vector<uintptr_t> mg_key(const agx_mesh *m) {
   return k;
 }
 
-static double norm_dv(const agx_mesh *m) { return m->rdx_blk * m->rdy_blk * m->rdz_blk; }
-
 int mg_solve_head(agx_mesh *m) {
   if (m->mp_on) solve_load_b(m);
   else solve_load(m);
@@ -3032,12 +3037,46 @@ void mg_solve_gated(agx_mesh *m, int k, std::vector<MGSnap> &snaps) {
   snaps.push_back(mg_snap(m));
   m->gate = reinterpret_cast<const int *>(reinterpret_cast<const char *>(m->gatedev) + offsetof(MGGate, closed));
   for (int i = 0; i < k; ++i) {
-    loop_step(m);
-    hipLaunchKernelGGL(k_mg_gate_check, dim3(1), dim3(64), 0, m->stream, m->gatedev, m->scal, norm_dv(m),
-                       mesh_volume(m->d), m->mg_eps);
+    loop_step(m);   // ends with k_mg_final_check
     snaps.push_back(mg_snap(m));
   }
   m->gate = nullptr;
+}
+
+// SolveIterative (multigrid_driver.cpp:721-755) for an eager solve, by gated passes: the host
+// enqueues several V-cycles at a time and reads the gate after them, instead of the norm after
+// each, as a pass behind the closed gate costs the GPU 2 us a launch and a norm read by the
+// host leaves it idle for 25 to 35 us.  The first four, then as many as the norm's rate so far
+// leaves to the threshold (at most MG_AHEAD).
+constexpr int MG_AHEAD = 16;
+static int iterate(agx_mesh *m, int &iters, double &def) {
+  first_defect_sum(m);
+  hipLaunchKernelGGL(k_mg_gate_open, dim3(1), dim3(64), 0, m->stream, m->gatedev, m->scal, norm_dv(m),
+                     mesh_volume(m->d), m->mg_eps);
+  std::vector<MGSnap> snaps;
+  iters = 0;
+  double before = 0.0;   // the norm before the last chunk (not read before the first)
+  for (int k = 4;;) {
+    mg_solve_gated(m, k, snaps);
+    hipError_t e = hipMemcpyAsync(m->gatehost, m->gatedev, sizeof(MGGate), hipMemcpyDeviceToHost, m->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
+    if (e != hipSuccess) return hip_fail(e, "mg_solve");
+    const MGGate gs = *m->gatehost;
+    const int ran = gs.iters - iters;
+    if (ran < 0 || ran > k) {
+      set_error("multigrid loop reports %d V-cycles of %d", ran, k);
+      return -70;
+    }
+    mg_restore(m, snaps[ran]);
+    iters = gs.iters;
+    def = gs.def;
+    if (gs.closed) return 0;
+    const double rate = before > 0.0 ? std::pow(def / before, 1.0 / ran) : 0.0;
+    k = 4;
+    if (m->mg_eps > 0.0 && rate > 0.0 && rate < 1.0)
+      k = (int)std::min<double>(MG_AHEAD, std::max(1.0, std::ceil(std::log(m->mg_eps / def) / std::log(rate))));
+    before = def;
+  }
 }
 
 int mg_solve_settle(agx_mesh *m, int stage, const std::vector<MGSnap> &snaps) {
