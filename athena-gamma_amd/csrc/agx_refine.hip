@@ -302,19 +302,27 @@ k_ref_prolong_fc_shared(RG r, const double *__restrict__ coarse, agx_ref_coords 
 // each 2x2x2 group of fine cells from its 24 outer faces; groups share no written face.
 // ProlongateInternalField for the 2x2x2 fine group of coarse cell (k, j, i) of block fb:
 // the 12 faces inside the group from its 24 outer faces (mesh_refinement.cpp:831-946).
-__device__ __forceinline__ void
-internal_group(const RG &r, double *__restrict__ b1, double *__restrict__ b2, double *__restrict__ b3,
-               const double *__restrict__ d1, const double *__restrict__ d2, const double *__restrict__ d3, int fb,
-               int i, int j, int k) {
-    const int fi = (i - r.cis) * 2 + r.is, fj = (j - r.cjs) * 2 + r.js, fk = (k - r.cks) * 2 + r.ks;
-    auto B1 = [&](int kk, int jj, int ii) -> double & { return b1[bx(r, r.n3, r.n2, r.n1 + 1, 1, fb, 0, kk, jj, ii)]; };
-    auto B2 = [&](int kk, int jj, int ii) -> double & { return b2[bx(r, r.n3, r.n2 + 1, r.n1, 1, fb, 0, kk, jj, ii)]; };
-    auto B3 = [&](int kk, int jj, int ii) -> double & { return b3[bx(r, r.n3 + 1, r.n2, r.n1, 1, fb, 0, kk, jj, ii)]; };
-    // Face?Area(fk+a, fj+b, ii)
-    auto A1 = [&](int a, int b) { return d2[fj + b] * d3[fk + a]; };
-    auto A2 = [&](int a, int ii) { return d1[ii] * d3[fk + a]; };
-    auto A3 = [&](int b, int ii) { return d1[ii] * d2[fj + b]; };
-    double Uxx = 0.0, Vyy = 0.0, Wzz = 0.0, Uxyz = 0.0, Vxyz = 0.0, Wxyz = 0.0;
+// Group holds the sums over the outer faces that every inner face uses; x1(a, b), x2(a, c) and
+// x3(b, c) are the inner faces at k offset a, j offset b, i offset c.
+struct Group {
+  const RG &r;
+  const double *b1, *b2, *b3, *d1, *d2, *d3;
+  int fb, fi, fj, fk;
+  double Uxx = 0.0, Vyy = 0.0, Wzz = 0.0, Uxyz = 0.0, Vxyz = 0.0, Wxyz = 0.0, Sdx1, Sdx2, Sdx3;
+  __device__ __forceinline__ int64_t i1(int kk, int jj, int ii) const { return bx(r, r.n3, r.n2, r.n1 + 1, 1, fb, 0, kk, jj, ii); }
+  __device__ __forceinline__ int64_t i2(int kk, int jj, int ii) const { return bx(r, r.n3, r.n2 + 1, r.n1, 1, fb, 0, kk, jj, ii); }
+  __device__ __forceinline__ int64_t i3(int kk, int jj, int ii) const { return bx(r, r.n3 + 1, r.n2, r.n1, 1, fb, 0, kk, jj, ii); }
+  __device__ __forceinline__ double B1(int kk, int jj, int ii) const { return b1[i1(kk, jj, ii)]; }
+  __device__ __forceinline__ double B2(int kk, int jj, int ii) const { return b2[i2(kk, jj, ii)]; }
+  __device__ __forceinline__ double B3(int kk, int jj, int ii) const { return b3[i3(kk, jj, ii)]; }
+  // Face?Area(fk+a, fj+b, ii)
+  __device__ __forceinline__ double A1(int a, int b) const { return d2[fj + b] * d3[fk + a]; }
+  __device__ __forceinline__ double A2(int a, int ii) const { return d1[ii] * d3[fk + a]; }
+  __device__ __forceinline__ double A3(int b, int ii) const { return d1[ii] * d2[fj + b]; }
+  __device__ __forceinline__ Group(const RG &r_, const double *b1_, const double *b2_, const double *b3_,
+                                   const double *d1_, const double *d2_, const double *d3_, int fb_, int i, int j, int k)
+      : r(r_), b1(b1_), b2(b2_), b3(b3_), d1(d1_), d2(d2_), d3(d3_), fb(fb_), fi((i - r.cis) * 2 + r.is),
+        fj((j - r.cjs) * 2 + r.js), fk((k - r.cks) * 2 + r.ks) {
 #pragma unroll
     for (int jj = 0; jj < 2; ++jj) {
       const int js = 2 * jj - 1, fjj = fj + jj, fjp = fj + 2 * jj;
@@ -333,38 +341,43 @@ internal_group(const RG &r, double *__restrict__ b1, double *__restrict__ b2, do
       }
     }
     const double s1 = d1[fi] + d1[fi + 1], s2 = d2[fj] + d2[fj + 1], s3 = d3[fk] + d3[fk + 1];
-    const double Sdx1 = s1 * s1, Sdx2 = s2 * s2, Sdx3 = s3 * s3;
+    Sdx1 = s1 * s1; Sdx2 = s2 * s2; Sdx3 = s3 * s3;
     Uxx *= 0.125; Vyy *= 0.125; Wzz *= 0.125;
     Uxyz *= 0.125 / (Sdx2 + Sdx3);
     Vxyz *= 0.125 / (Sdx1 + Sdx3);
     Wxyz *= 0.125 / (Sdx1 + Sdx2);
+  }
+  __device__ __forceinline__ double x1(int a, int b) const {
+    double v = 0.5 * (B1(fk + a, fj + b, fi) * A1(a, b) + B1(fk + a, fj + b, fi + 2) * A1(a, b)) + Uxx;
+    v = a ? v + Sdx3 * Vxyz : v - Sdx3 * Vxyz;
+    v = b ? v + Sdx2 * Wxyz : v - Sdx2 * Wxyz;
+    return v / A1(a, b);
+  }
+  __device__ __forceinline__ double x2(int a, int c) const {
+    double v = 0.5 * (B2(fk + a, fj, fi + c) * A2(a, fi + c) + B2(fk + a, fj + 2, fi + c) * A2(a, fi + c)) + Vyy;
+    v = a ? v + Sdx3 * Uxyz : v - Sdx3 * Uxyz;
+    v = c ? v + Sdx1 * Wxyz : v - Sdx1 * Wxyz;
+    return v / A2(a, fi + c);
+  }
+  __device__ __forceinline__ double x3(int b, int c) const {
+    double v = 0.5 * (B3(fk + 2, fj + b, fi + c) * A3(b, fi + c) + B3(fk, fj + b, fi + c) * A3(b, fi + c)) + Wzz;
+    v = b ? v + Sdx2 * Uxyz : v - Sdx2 * Uxyz;
+    v = c ? v + Sdx1 * Vxyz : v - Sdx1 * Vxyz;
+    return v / A3(b, fi + c);
+  }
+};
+__device__ __forceinline__ void
+internal_group(const RG &r, double *__restrict__ b1, double *__restrict__ b2, double *__restrict__ b3,
+               const double *__restrict__ d1, const double *__restrict__ d2, const double *__restrict__ d3, int fb,
+               int i, int j, int k) {
+  const Group g(r, b1, b2, b3, d1, d2, d3, fb, i, j, k);
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        double v = 0.5 * (B1(fk + a, fj + b, fi) * A1(a, b) + B1(fk + a, fj + b, fi + 2) * A1(a, b)) + Uxx;
-        v = a ? v + Sdx3 * Vxyz : v - Sdx3 * Vxyz;
-        v = b ? v + Sdx2 * Wxyz : v - Sdx2 * Wxyz;
-        B1(fk + a, fj + b, fi + 1) = v / A1(a, b);
-      }
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        double v = 0.5 * (B2(fk + a, fj, fi + c) * A2(a, fi + c) + B2(fk + a, fj + 2, fi + c) * A2(a, fi + c)) + Vyy;
-        v = a ? v + Sdx3 * Uxyz : v - Sdx3 * Uxyz;
-        v = c ? v + Sdx1 * Wxyz : v - Sdx1 * Wxyz;
-        B2(fk + a, fj + 1, fi + c) = v / A2(a, fi + c);
-      }
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        double v = 0.5 * (B3(fk + 2, fj + b, fi + c) * A3(b, fi + c) + B3(fk, fj + b, fi + c) * A3(b, fi + c)) + Wzz;
-        v = b ? v + Sdx2 * Uxyz : v - Sdx2 * Uxyz;
-        v = c ? v + Sdx1 * Vxyz : v - Sdx1 * Vxyz;
-        B3(fk + 1, fj + b, fi + c) = v / A3(b, fi + c);
-      }
+  for (int e = 0; e < 4; ++e) {
+    const int p = e >> 1, q = e & 1;
+    b1[g.i1(g.fk + p, g.fj + q, g.fi + 1)] = g.x1(p, q);
+    b2[g.i2(g.fk + p, g.fj + 1, g.fi + q)] = g.x2(p, q);
+    b3[g.i3(g.fk + 1, g.fj + p, g.fi + q)] = g.x3(p, q);
+  }
 }
 
 __device__ __forceinline__ void
@@ -392,20 +405,13 @@ k_ref_prolong_fc_internal(RG r, double *__restrict__ b1, double *__restrict__ b2
 // Field::CalculateCellCenteredField, uniform branch (field.cpp:112-176: lw = rw = 0.5), then
 // EquationOfState::PrimitiveToConserved (adiabatic_mhd.cpp:99-136; isothermal_mhd.cpp:
 // 82-108 without energy) on the fine cells of each coarse range.
-// bcc and u of fine cell (k, j, i) of block fb from its faces and w (the loop body of
+// bcc and u of fine cell (k, j, i) of block fb from its bcc and w (the loop body of
 // CalculateCellCenteredField + PrimitiveToConserved)
 template <bool ISO>
 __device__ __forceinline__ void
-p2c_cell(const RG &r, const double *__restrict__ w, const double *__restrict__ b1, const double *__restrict__ b2,
-         const double *__restrict__ b3, double *__restrict__ bcc, double *__restrict__ u, double igm1, int fb, int i,
-         int j, int k) {
+p2c_store(const RG &r, const double *__restrict__ w, double bc1, double bc2, double bc3, double *__restrict__ bcc,
+          double *__restrict__ u, double igm1, int fb, int i, int j, int k) {
   constexpr int NH = ISO ? 4 : 5;
-    const double bc1 = 0.5 * b1[bx(r, r.n3, r.n2, r.n1 + 1, 1, fb, 0, k, j, i)] +
-                       0.5 * b1[bx(r, r.n3, r.n2, r.n1 + 1, 1, fb, 0, k, j, i + 1)];
-    const double bc2 = 0.5 * b2[bx(r, r.n3, r.n2 + 1, r.n1, 1, fb, 0, k, j, i)] +
-                       0.5 * b2[bx(r, r.n3, r.n2 + 1, r.n1, 1, fb, 0, k, j + 1, i)];
-    const double bc3 = 0.5 * b3[bx(r, r.n3 + 1, r.n2, r.n1, 1, fb, 0, k, j, i)] +
-                       0.5 * b3[bx(r, r.n3 + 1, r.n2, r.n1, 1, fb, 0, k + 1, j, i)];
     bcc[bx(r, r.n3, r.n2, r.n1, 3, fb, 0, k, j, i)] = bc1;
     bcc[bx(r, r.n3, r.n2, r.n1, 3, fb, 1, k, j, i)] = bc2;
     bcc[bx(r, r.n3, r.n2, r.n1, 3, fb, 2, k, j, i)] = bc3;
@@ -422,6 +428,20 @@ p2c_cell(const RG &r, const double *__restrict__ w, const double *__restrict__ b
       u[bx(r, r.n3, r.n2, r.n1, NH, fb, 4, k, j, i)] =
           w_p * igm1 + 0.5 * (w_d * (w_vx * w_vx + w_vy * w_vy + w_vz * w_vz) + (bc1 * bc1 + bc2 * bc2 + bc3 * bc3));
     }
+}
+
+template <bool ISO>
+__device__ __forceinline__ void
+p2c_cell(const RG &r, const double *__restrict__ w, const double *__restrict__ b1, const double *__restrict__ b2,
+         const double *__restrict__ b3, double *__restrict__ bcc, double *__restrict__ u, double igm1, int fb, int i,
+         int j, int k) {
+  const double bc1 = 0.5 * b1[bx(r, r.n3, r.n2, r.n1 + 1, 1, fb, 0, k, j, i)] +
+                     0.5 * b1[bx(r, r.n3, r.n2, r.n1 + 1, 1, fb, 0, k, j, i + 1)];
+  const double bc2 = 0.5 * b2[bx(r, r.n3, r.n2 + 1, r.n1, 1, fb, 0, k, j, i)] +
+                     0.5 * b2[bx(r, r.n3, r.n2 + 1, r.n1, 1, fb, 0, k, j + 1, i)];
+  const double bc3 = 0.5 * b3[bx(r, r.n3 + 1, r.n2, r.n1, 1, fb, 0, k, j, i)] +
+                     0.5 * b3[bx(r, r.n3 + 1, r.n2, r.n1, 1, fb, 0, k + 1, j, i)];
+  p2c_store<ISO>(r, w, bc1, bc2, bc3, bcc, u, igm1, fb, i, j, k);
 }
 
 template <bool ISO>
@@ -533,9 +553,13 @@ k_ref_prolong_all(RG r, int nvar, const double *__restrict__ cw, const double *_
   else if (l == 3) b_ref_prolong_fc_shared<2>(r, cb3, cc, b3, fc, sp.p[3][y]);
 }
 
-// ProlongateInternalField, then CalculateCellCenteredField + PrimitiveToConserved, per
-// 2x2x2 group: the thread that forms a group's 12 inner faces then converts its 8 cells,
-// whose other faces are the group's outer (shared) faces, final before this launch.
+// ProlongateInternalField, then CalculateCellCenteredField + PrimitiveToConserved, one thread per
+// fine cell, eight adjacent lanes per 2x2x2 group.  Each forms the group's sums from its 24 outer
+// (shared) faces, final before this launch, which the eight read together; then the cell's three
+// inner faces, each of which one of its two cells stores; then converts the cell from these
+// values.  No value is read back, where one thread per group stored its 12 faces and went through
+// its 8 cells one load latency after another.  Three levels of 16^3 blocks (14 launches a cycle):
+// 17.0 -> 9.8 us a launch; bound by the latency of those loads.
 template <bool ISO>
 __global__ void __launch_bounds__(RBS)
 k_ref_internal_p2c(RG r, double *__restrict__ b1, double *__restrict__ b2, double *__restrict__ b3,
@@ -547,15 +571,22 @@ k_ref_internal_p2c(RG r, double *__restrict__ b1, double *__restrict__ b2, doubl
   const int fb = it.fb;
   const double *d1 = fc.dx1f + (int64_t)fb * r.n1, *d2 = fc.dx2f + (int64_t)fb * r.n2,
                *d3 = fc.dx3f + (int64_t)fb * r.n3;
-  for (unsigned t = first_t(); t < cnt; t += stride_t()) {
+  const int e = threadIdx.x & 7, c = e & 1, b = (e >> 1) & 1, a = e >> 2;   // the cell's place in its group
+  for (unsigned t = first_t() >> 3; t < cnt; t += stride_t() >> 3) {
     const int i = q.si + (int)(t % (unsigned)q.w1);
     const unsigned s = t / (unsigned)q.w1;
     const int j = q.sj + (int)(s % (unsigned)q.w2), k = q.sk + (int)(s / (unsigned)q.w2);
-    internal_group(r, b1, b2, b3, d1, d2, d3, fb, i, j, k);
-    const int fi = (i - r.cis) * 2 + r.is, fj = (j - r.cjs) * 2 + r.js, fk = (k - r.cks) * 2 + r.ks;
-#pragma unroll
-    for (int c = 0; c < 8; ++c)
-      p2c_cell<ISO>(r, w, b1, b2, b3, bcc, u, igm1, fb, fi + (c & 1), fj + ((c >> 1) & 1), fk + (c >> 2));
+    const Group g(r, b1, b2, b3, d1, d2, d3, fb, i, j, k);
+    const double v1 = g.x1(a, b), v2 = g.x2(a, c), v3 = g.x3(b, c);
+    // the cell's outer face in each direction; lower and upper as p2c_cell adds them
+    const double o1 = g.B1(g.fk + a, g.fj + b, g.fi + 2 * c), o2 = g.B2(g.fk + a, g.fj + 2 * b, g.fi + c),
+                 o3 = g.B3(g.fk + 2 * a, g.fj + b, g.fi + c);
+    const double bc1 = 0.5 * (c ? v1 : o1) + 0.5 * (c ? o1 : v1), bc2 = 0.5 * (b ? v2 : o2) + 0.5 * (b ? o2 : v2),
+                 bc3 = 0.5 * (a ? v3 : o3) + 0.5 * (a ? o3 : v3);
+    if (c == 0) b1[g.i1(g.fk + a, g.fj + b, g.fi + 1)] = v1;
+    if (b == 0) b2[g.i2(g.fk + a, g.fj + 1, g.fi + c)] = v2;
+    if (a == 0) b3[g.i3(g.fk + 1, g.fj + b, g.fi + c)] = v3;
+    p2c_store<ISO>(r, w, bc1, bc2, bc3, bcc, u, igm1, fb, g.fi + c, g.fj + b, g.fk + a);
   }
 }
 
@@ -1368,10 +1399,10 @@ int agx_ref_internal_to_cons(const agx_ref_list *l, double *b1f, double *b2f, do
   if (l->nitems == 0) return 0;
   const double igm1 = iso ? 0.0 : 1.0 / (gamma - 1.0);
   if (iso)
-    hipLaunchKernelGGL(k_ref_internal_p2c<true>, dim3(l->G, l->nitems), dim3(RBS), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(k_ref_internal_p2c<true>, dim3(std::min(64, 8 * l->G), l->nitems), dim3(RBS), 0, (hipStream_t)stream,
                        make_rg(l->g), b1f, b2f, b3f, fc, w, bcc, u, igm1, l->items);
   else
-    hipLaunchKernelGGL(k_ref_internal_p2c<false>, dim3(l->G, l->nitems), dim3(RBS), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(k_ref_internal_p2c<false>, dim3(std::min(64, 8 * l->G), l->nitems), dim3(RBS), 0, (hipStream_t)stream,
                        make_rg(l->g), b1f, b2f, b3f, fc, w, bcc, u, igm1, l->items);
   return launch_status("agx_ref_internal_to_cons");
 }
