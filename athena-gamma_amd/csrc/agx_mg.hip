@@ -369,6 +369,49 @@ k_mg_partial(const int *__restrict__ gate, const T *__restrict__ a, const T *__r
   if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
+// k_mg_partial's mode 1 with a thread's cells as (i, i+1) pairs of a row (n1 even), read as one
+// vector, and stepped from pair to pair without divisions, which were most of its instructions:
+// 256^3 FP64 93 -> 66 us, 4.0 TB/s of u and source.  Each thread sums its own pairs, so the order
+// differs from mode 1's, which runs where n1 is odd.
+template <typename T>
+__global__ void __launch_bounds__(BS)
+k_mg_norm_pairs(const int *__restrict__ gate, const T *__restrict__ u, const T *__restrict__ src, int n1, int n2,
+                int n3, T idx2, double *__restrict__ part) {
+  if (gate && *gate) return;   // a closed gate: the recorded V-cycle loop has ended
+  using V = typename Vec2<T>::type;
+  __shared__ double sh[BS];
+  const unsigned nh = (unsigned)n1 >> 1;
+  unsigned t0, t1;
+  wg_range(nh * (unsigned)n2 * (unsigned)n3, t0, t1);
+  const unsigned dh = BS % nh, dr = BS / nh;   // a step: pairs along the row, rows
+  const unsigned dj = dr % (unsigned)n2, dk = dr / (unsigned)n2;
+  unsigned t = t0 + threadIdx.x;
+  unsigned h = t % nh, r = t / nh, j = r % (unsigned)n2, k = r / (unsigned)n2;
+  double v = 0.0;
+  for (; t < t1; t += BS) {
+    const int64_t row = LIX(n1, n2, k, j, 0);
+    const T *c = u + row + 2 * h;
+    const V uc = load2(c, 0), f = load2(src, row + 2 * h);
+    const V kp = load2(u, LIX(n1, n2, wrapp(k, n3), j, 2 * h)), km = load2(u, LIX(n1, n2, wrapm(k, n3), j, 2 * h));
+    const V jp = load2(u, LIX(n1, n2, k, wrapp(j, n2), 2 * h)), jm = load2(u, LIX(n1, n2, k, wrapm(j, n2), 2 * h));
+    const T im = u[row + (h == 0 ? n1 - 1 : 2 * (int)h - 1)], ip = u[row + (h == nh - 1 ? 0 : 2 * h + 2)];
+    const double d0 = (T(6.0) * uc.x - kp.x - jp.x - uc.y - km.x - jm.x - im) * idx2 + f.x;
+    const double d1 = (T(6.0) * uc.y - kp.y - jp.y - ip - km.y - jm.y - uc.x) * idx2 + f.y;
+    v += d0 * d0;
+    v += d1 * d1;
+    h += dh; j += dj; k += dk;
+    if (h >= nh) { h -= nh; ++j; }
+    if (j >= (unsigned)n2) { j -= n2; ++k; }
+  }
+  sh[threadIdx.x] = v;
+  __syncthreads();
+  for (int s = BS / 2; s > 0; s >>= 1) {
+    if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+}
+
 // the sum of n partials, in thread 0 (fixed order)
 __device__ __forceinline__ double part_sum(const double *__restrict__ part, int64_t n) {
   __shared__ double sh[BS];
@@ -2671,7 +2714,11 @@ static void level_sum(agx_mesh *m, std::vector<MGLevelT<T>> &H, int l, int mode,
   if (mode == 0)
     hipLaunchKernelGGL((k_mg_partial<0, T>), dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, L.u, L.src, L.n1,
                        L.n2, L.n3, T(idx2), m->red);
-  else
+  else if ((L.n1 & 1) == 0) {
+    nb = npart(lcells(L) / 2);
+    hipLaunchKernelGGL(k_mg_norm_pairs<T>, dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, L.u, L.src, L.n1,
+                       L.n2, L.n3, T(idx2), m->red);
+  } else
     hipLaunchKernelGGL((k_mg_partial<1, T>), dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, L.u, L.src, L.n1,
                        L.n2, L.n3, T(idx2), m->red);
   final_sum(m, nb, slot);

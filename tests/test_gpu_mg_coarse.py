@@ -5,7 +5,7 @@ chunks that end inside; the same potential bit for bit."""
 import numpy as np
 import pytest
 
-from oracle.orc import make_desc
+from oracle.orc import Oracle, make_desc
 from tests.test_gpu_mg_levels import vcycle_by_steps
 
 pytestmark = pytest.mark.gpu
@@ -78,3 +78,22 @@ def test_periodic_passes_identical(agx, n, b, precision):
         out.append((m.get("phi"), m.mg_last()))
         m.close()
     assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
+
+
+@pytest.mark.parametrize("n,b", [((4, 4, 4), 4), ((36, 20, 12), 4), ((64, 4, 8), 4), ((24, 40, 56), 8), ((48, 96, 16), 16)])
+def test_defect_norm_matches_oracle(agx, n, b):
+    """the finest defect's norm, rows shorter and longer than a workgroup's step: sums of at most
+    2e5 squares in another order agree to 1e-9 of the norm (the bar of the parity tests)"""
+    h = 1.0 / max(n)
+    d = make_desc(nx=n, bnx=(b, b, b), box=tuple((0.0, h * q) for q in n), self_gravity=1, mg_bc=0, mg_mode=0,
+                  four_pi_G=1.0, mg_threshold=-1.0, mg_niter=1)
+    U = np.zeros((5, n[2], n[1], n[0]))
+    U[0] = np.random.default_rng(6).uniform(0.5, 1.5, n[::-1])
+    ub = agx.scatter_cells(d, U)
+    norms = []
+    for m in (agx.Mesh(d), Oracle(d)):
+        m.set("u", ub)
+        m.mg_solve(0)
+        norms.append(m.mg_last()[0])
+    print(n, norms, flush=True)
+    assert abs(norms[0] - norms[1]) <= 1e-9 * norms[1]
