@@ -127,6 +127,7 @@ struct MGGate {
   int closed;
   int iters;     // V-cycles the loop has run
   double def;    // defect norm after the last of them (before the loop: the first norm)
+  double first;  // the norm before the loop
 };
 
 // Host-side multigrid state that a V-cycle changes: the red-black offset, the level
@@ -200,7 +201,7 @@ struct agx_mesh {
   agx::MGGate *gatedev = nullptr;    // gate of a recorded threshold loop (device)
   agx::MGGate *gatehost = nullptr;   // its pinned host mirror
   const int *gate = nullptr;         // &gatedev->closed while a gated loop is enqueued, else null
-  int mg_kpred[2] = {-1, -1};        // V-cycles of the last threshold solve of each stage
+  int mg_kpred[3] = {-1, -1, -1};    // V-cycles of the last threshold solve of stage 0 (a solve by itself), 1, 2
   std::vector<agx::MGLevel> lev;
   std::vector<agx::MGLevel32> lev32;   // mixed precision only
   double *mgpool = nullptr;

@@ -440,6 +440,7 @@ __global__ void k_mg_gate_open(MGGate *g, const double *__restrict__ scal, doubl
   const double def = sqrt(scal[0] * dv / vol);
   g->iters = 0;
   g->def = def;
+  g->first = def;
   g->closed = (def > eps) ? 0 : 1;
 }
 
@@ -1947,7 +1948,7 @@ static int64_t pad32(int64_t n) { return (n + 63) / 64 * 64; }   // 64 elements:
 static int64_t npart(int64_t n) { return std::min<int64_t>(grid1d(n, BS), NPART); }
 
 static double finish_norm(agx_mesh *m);
-static int iterate(agx_mesh *m, int &iters, double &def);
+static int iterate(agx_mesh *m, int stage, int &iters, double &def);
 static void first_defect_sum(agx_mesh *m);
 static void loop_step(agx_mesh *m);
 static double mesh_volume(const agx_mesh_desc &d);
@@ -2500,10 +2501,10 @@ static int mg_solve_b(agx_mesh *m, int stage) {
   int iters = 0;
   double def = 0.0;
   if (m->mg_eps >= 0.0) {   // SolveIterative, multigrid_driver.cpp:721-755
-    int rc = iterate(m, iters, def);
+    int rc = iterate(m, stage, iters, def);
     if (rc) return rc;
     m->last_norm = def;
-    if (stage == 1 || stage == 2) m->mg_kpred[stage - 1] = iters;
+    if (stage >= 0 && stage <= 2) m->mg_kpred[stage] = iters;
   } else {   // SolveIterativeFixedTimes, multigrid_driver.cpp:762-771
     for (int n = 0; n < m->mg_niter; ++n) {
       if (m->mixed) correction_step_b(m);
@@ -3009,10 +3010,10 @@ int mg_solve(agx_mesh *m, int stage) {
   int iters = 0;
   double def = 0.0;
   if (m->mg_eps >= 0.0) {   // SolveIterative, multigrid_driver.cpp:721-755
-    int rc = iterate(m, iters, def);
+    int rc = iterate(m, stage, iters, def);
     if (rc) return rc;
     m->last_norm = def;
-    if (stage == 1 || stage == 2) m->mg_kpred[stage - 1] = iters;
+    if (stage >= 0 && stage <= 2) m->mg_kpred[stage] = iters;
     subtract_average(m, 1);
   } else {   // SolveIterativeFixedTimes, multigrid_driver.cpp:762-771
     if (mixed && m->mg_niter > 0) defect_to32(m, false);
@@ -3090,20 +3091,65 @@ void mg_solve_gated(agx_mesh *m, int k, std::vector<MGSnap> &snaps) {
   m->gate = nullptr;
 }
 
-// SolveIterative (multigrid_driver.cpp:721-755) for an eager solve, by gated passes: the host
-// enqueues several V-cycles at a time and reads the gate after them, instead of the norm after
-// each, as a pass behind the closed gate costs the GPU 2 us a launch and a norm read by the
-// host leaves it idle for 25 to 35 us.  The first four, then as many as the norm's rate so far
-// leaves to the threshold (at most MG_AHEAD).
-constexpr int MG_AHEAD = 16;
-static int iterate(agx_mesh *m, int &iters, double &def) {
+// SolveIterative's loop (multigrid_driver.cpp:733-753) from the iters-th V-cycle on, the host
+// reading the norm after each
+static void iterate_checked(agx_mesh *m, int &iters, double &def) {
+  int n = iters;
+  while (def > m->mg_eps) {
+    loop_step(m);
+    iters++;
+    double olddef = def;
+    def = finish_norm(m);
+    if (def / olddef > 0.8) {
+      if (m->mg_eps == 0.0) break;
+    }
+    if (n > 100) break;
+    n++;
+  }
+}
+
+// launches of one pass of the loop (loop_step)
+static int pass_launches(const agx_mesh *m) {
+  const bool mp = m->mp_on;
+  const int ct = mp ? coarse_top_b(m) : coarse_top(m->lev);   // by the sizes alone: the FP32 levels' too
+  const int ni = std::max(m->g.nb1, std::max(m->g.nb2, m->g.nb3)) >> (m->nrootlevel - 1);
+  int n = 2 + (mp && m->mixed ? 4 : 0);   // the norm; correction_step_b's steps around its V-cycle
+  if (ct >= 0) n += 1;
+  else n += mp ? 2 + 4 * ni : (ni == 1 ? 1 : 6 + 2 * ni);
+  for (int l = std::max(ct, 0) + 1; l < m->ntotal; ++l)
+    n += ((mp ? m->mg_coarse != 0 : m->mg_fuse != 0) && pass_level(m->lev[l])) ? 2 : (mp ? 14 : 6);
+  return n;
+}
+
+// SolveIterative (multigrid_driver.cpp:721-755) for an eager solve.  A norm that the host reads
+// leaves the GPU idle for 25 to 35 us, so the host enqueues gated passes, as many as the norm's
+// rate leaves whole V-cycles to the threshold (at most MG_AHEAD), and reads the gate after them.
+// A pass behind the closed gate costs 2 us a launch, so
+// - a solve reads the norm before the loop and after its first V-cycle, as it may need no more,
+//   unless the stage's last solve took four or more (us a solve, 64^3: none needed 303 periodic FMG
+//   and 69 from the last potential, with four passes enqueued unread 324 and 157);
+// - passes of many launches keep the read after each (one a step with multipole boundaries, 100
+//   launches: none needed 1130, with four passes unread 2460), and timed ones, whose launch counts
+//   would hold the closed passes.
+constexpr int MG_AHEAD = 16, MG_AHEAD_LAUNCHES = 56;
+static int iterate(agx_mesh *m, int stage, int &iters, double &def) {
   first_defect_sum(m);
+  iters = 0;
+  const bool each = m->timer.enabled || pass_launches(m) > MG_AHEAD_LAUNCHES;
+  int k = (!each && stage >= 0 && stage <= 2 && m->mg_kpred[stage] >= 4) ? 2 : 1;
+  def = 0.0;   // not read yet
+  if (k == 1) {
+    def = finish_norm(m);
+    if (!(def > m->mg_eps)) return 0;
+    if (each) {
+      iterate_checked(m, iters, def);
+      return 0;
+    }
+  }
   hipLaunchKernelGGL(k_mg_gate_open, dim3(1), dim3(64), 0, m->stream, m->gatedev, m->scal, norm_dv(m),
                      mesh_volume(m->d), m->mg_eps);
   std::vector<MGSnap> snaps;
-  iters = 0;
-  double before = 0.0;   // the norm before the last chunk (not read before the first)
-  for (int k = 4;;) {
+  for (;;) {
     mg_solve_gated(m, k, snaps);
     hipError_t e = hipMemcpyAsync(m->gatehost, m->gatedev, sizeof(MGGate), hipMemcpyDeviceToHost, m->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
@@ -3115,14 +3161,15 @@ static int iterate(agx_mesh *m, int &iters, double &def) {
       return -70;
     }
     mg_restore(m, snaps[ran]);
+    const double before = iters ? def : gs.first;
     iters = gs.iters;
     def = gs.def;
     if (gs.closed) return 0;
-    const double rate = before > 0.0 ? std::pow(def / before, 1.0 / ran) : 0.0;
-    k = 4;
-    if (m->mg_eps > 0.0 && rate > 0.0 && rate < 1.0)
-      k = (int)std::min<double>(MG_AHEAD, std::max(1.0, std::ceil(std::log(m->mg_eps / def) / std::log(rate))));
-    before = def;
+    const double rate = std::pow(def / before, 1.0 / ran);   // an open gate: the whole chunk ran
+    if (m->mg_eps == 0.0) k = 4;   // runs to the rounding floor, which no rate foretells
+    else if (rate > 0.0 && rate < 1.0)
+      k = (int)std::min<double>(MG_AHEAD, std::max(1.0, std::floor(std::log(m->mg_eps / def) / std::log(rate))));
+    else k = 1;
   }
 }
 
@@ -3138,23 +3185,10 @@ int mg_solve_settle(agx_mesh *m, int stage, const std::vector<MGSnap> &snaps) {
   mg_restore(m, snaps[gs.iters]);
   double def = gs.def;
   int iters = gs.iters;
-  if (!gs.closed) {   // the recorded passes ended before the loop did: go on as mg_solve
-    int n = iters;
-    while (def > m->mg_eps) {
-      loop_step(m);
-      iters++;
-      double olddef = def;
-      def = finish_norm(m);
-      if (def / olddef > 0.8) {
-        if (m->mg_eps == 0.0) break;
-      }
-      if (n > 100) break;
-      n++;
-    }
-  }
+  if (!gs.closed) iterate_checked(m, iters, def);   // the recorded passes ended before the loop did
   m->last_norm = def;
   m->last_iters = iters;
-  if (stage == 1 || stage == 2) m->mg_kpred[stage - 1] = iters;
+  if (stage >= 0 && stage <= 2) m->mg_kpred[stage] = iters;
   return 0;
 }
 

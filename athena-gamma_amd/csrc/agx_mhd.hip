@@ -3885,7 +3885,7 @@ static int cycle_graphs_threshold(agx_mesh *m, double tlim, int32_t ncycles, int
   int rc = push_scalars(m, tlim);
   while (!rc && n < ncycles && m->time < tlim) {
     for (int seg = 0; seg < 3 && !rc; ++seg) {
-      const int k = seg < 2 ? std::max(m->mg_kpred[seg], 0) : 0;
+      const int k = seg < 2 ? std::max(m->mg_kpred[seg + 1], 0) : 0;
       int idx = -1;
       rc = graph_for_segment(m, seg, k, &idx);
       if (rc) break;
