@@ -1324,14 +1324,14 @@ struct FluxArgs {
   uint8_t *nearf;                          // near-tie flags of FP32 PPM, nflag bytes per direction
   int64_t nflag;
   int dir0, ndir;                          // the launch's directions
+  int xcd;                                 // workgroups in the XCD-aware order
 };
-template <typename P>
-__device__ __forceinline__ P of_dir(P const (&p)[3], int dir) { return dir == 0 ? p[0] : (dir == 1 ? p[1] : p[2]); }
 
-// One face of Hydro::CalculateFluxes in direction dir: face_flux at (b, id), written to
+// One face of Hydro::CalculateFluxes in direction DIR: face_flux at (b, id), written to
 // the face arrays; FLAG also writes the face's near-tie flag (0 or 1) to nearf.
-template <int ORDER, int RS, typename T, bool ISO, bool FLAG>
-__device__ __forceinline__ void flux_face(const Geo &g, const FluxArgs<T> &a, int dir, int b, int64_t id, int cidx) {
+template <int DIR, int ORDER, int RS, typename T, bool ISO, bool FLAG>
+__device__ __forceinline__ void flux_face(const Geo &g, const FluxArgs<T> &a, int b, int64_t id, int cidx) {
+  constexpr int dir = DIR;
   const int64_t sj = g.P, sk = (int64_t)g.J * g.P;   // strides along j, k
   const int64_t st = dir == 0 ? 1 : (dir == 1 ? sj : sk), st1 = dir == 0 ? sj : (dir == 1 ? sk : 1),
                 st2 = dir == 0 ? sk : (dir == 1 ? 1 : sj);
@@ -1340,33 +1340,51 @@ __device__ __forceinline__ void flux_face(const Geo &g, const FluxArgs<T> &a, in
   T f[5], fey, fez, fw;
   bool near;
   face_flux<ORDER, RS, T, ISO, FLAG>(dir, a.w + (int64_t)b * NHYDRO * g.S, a.bcc + (int64_t)b * 3 * g.S, g.S, id, st,
-                                     st1, st2, pc, g.PL, cidx, T(of_dir(a.bn, dir)[fo]), T(a.gamma), T(a.cs),
+                                     st1, st2, pc, g.PL, cidx, T(a.bn[dir][fo]), T(a.gamma), T(a.cs),
                                      T(a.dfl), T(a.pfl), T(a.coef[b].dx[dir]), T(*a.dtp), f, fey, fez, fw, &near);
   const int ivx = IVX + dir, ivy = IVX + (dir == 2 ? 0 : dir + 1), ivz = IVX + (dir == 0 ? 2 : dir - 1);
-  T *fb = of_dir(a.flx, dir) + (int64_t)b * NHYDRO * g.S + id;
+  T *fb = a.flx[dir] + (int64_t)b * NHYDRO * g.S + id;
   fb[IDN * g.S] = f[0];
   fb[ivx * g.S] = f[1];
   fb[ivy * g.S] = f[2];
   fb[ivz * g.S] = f[3];
   if (!ISO) fb[IEN * g.S] = f[4];
-  of_dir(a.ey, dir)[fo] = fey;
-  of_dir(a.ez, dir)[fo] = fez;
-  of_dir(a.wct, dir)[fo] = fw;
+  a.ey[dir][fo] = fey;
+  a.ez[dir][fo] = fez;
+  a.wct[dir][fo] = fw;
   if constexpr (FLAG) a.nearf[dir * a.nflag + fo] = near ? 1 : 0;
 }
 
+// Waves per SIMD asked of the compiler: FP64 characteristic PLM takes 176 registers, 2 waves, where
+// 168 with four spilled are 3 (256^3 in 64^3 blocks: 3.54 ms a launch, as three launches took); Roe and
+// LHLLD would spill 20 to 106.
+template <int ORDER, int RS, typename T>
+constexpr int flux_waves() {
+  return ORDER == ORDER_PLM_CHAR && sizeof(T) == 8 && (RS == AGX_RSOLVER_HLLD || RS == AGX_RSOLVER_HLLE) ? 3 : 1;
+}
+
 // Hydro::CalculateFluxes, one thread per face (face_flux), the directions of the launch in one
-// grid: a workgroup's direction is blockIdx.x mod ndir (in the XCD-aware order), so the three
-// directions of a piece of a plane run together and share its lines of w and bcc, and a small
-// mesh fills the chip once instead of three times.  Cycles in us, three launches against one
-// (with the time step's two launches made one, 4 us): 64 x 32 x 32 FP64 PLM 119 : 95, 64^3
-// 246 : 215, 120 x 90 x 70 PPM 913 : 883, 256^3 mixed 6797 : 6556.  Bound by FP64 and reciprocal
-// issue on large meshes.  For FP32 PPM nearf (one byte per cell of the block arrays and
-// direction) receives each face's near-tie flag.
+// grid: a workgroup's direction is blockIdx.x mod ndir, so the three directions of a piece of a
+// plane run together and share its lines of w and bcc, and a small mesh fills the chip once instead
+// of three times.  Cycles in us, three launches against one (with the time step's two launches made
+// one, 4 us): 64 x 32 x 32 FP64 PLM 119 : 95, 64^3 246 : 215, 120 x 90 x 70 PPM 913 : 883, 256^3 mixed
+// 6797 : 6556.  Bound by FP64 and reciprocal issue on large meshes.
+//
+// The face's arithmetic is compiled once for each direction behind a uniform branch: strides and
+// pointers picked at run time cost 2 to 4% of a large launch (us, 256^3 in 64^3 blocks, three
+// launches : one with the direction at run time : compiled; FP64 PLM 2590 : 2650 : 2485, mixed PPM
+// 2730 : 2834 : 2730; one block of 256^3 FP64 donor cell 1738 : 1811 : 1712, PLM 2230 : 2370 : 2285).
+// Those with the plain order of workgroups: XCD-aware, an XCD keeps a piece's neighbours and what the
+// stage kernel reads back, which pays while L2 and the last-level cache hold the arrays (cycles, plain :
+// XCD-aware; 32^3 mixed 92 : 83, 64^3 FP64 209 : 205), and beyond costs 1 to 3% (2553 for the 2485, 2788
+// for the 2730), so launch_flux draws the line at that cache.
+//
+// For FP32 PPM nearf (one byte per cell of the block arrays and direction) receives each face's
+// near-tie flag.
 template <int ORDER, int RS, typename T, bool ISO>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, (flux_waves<ORDER, RS, T>()))
 k_flux(Geo g, FluxArgs<T> a) {
-  const uint3 wg = xcd_block();
+  const uint3 wg = a.xcd ? xcd_block() : make_uint3(blockIdx.x, blockIdx.y, blockIdx.z);
   const int part = (int)(wg.x / (unsigned)a.ndir), dir = a.dir0 + (int)(wg.x - part * (unsigned)a.ndir);
   const int il = g.is - (dir != 0), jl = g.js - (dir != 1), k = g.ks - (dir != 2) + (int)wg.y, b = wg.z;
   const unsigned ni = g.ie + 1 - il + 1, nj = g.je + 1 - jl + 1, q = part * 256u + threadIdx.x;
@@ -1374,7 +1392,11 @@ k_flux(Geo g, FluxArgs<T> a) {
   const unsigned qj = q / ni;
   const int j = jl + (int)qj, i = il + (int)(q - qj * ni);
   const int cidx = dir == 0 ? i : (dir == 1 ? j : k);   // index of the cell above the face
-  flux_face<ORDER, RS, T, ISO, flux_flagged<ORDER, T>()>(g, a, dir, b, IDX(g, k, j, i), cidx);
+  const int64_t id = IDX(g, k, j, i);
+  constexpr bool F = flux_flagged<ORDER, T>();
+  if (dir == 0) flux_face<0, ORDER, RS, T, ISO, F>(g, a, b, id, cidx);
+  else if (dir == 1) flux_face<1, ORDER, RS, T, ISO, F>(g, a, b, id, cidx);
+  else flux_face<2, ORDER, RS, T, ISO, F>(g, a, b, id, cidx);
 }
 
 // Second pass of FP32 PPM fluxes: each workgroup scans FIX_SPAN bytes of nearf (16 per
@@ -1415,7 +1437,9 @@ k_flux_fix(Geo g, FluxArgs<float> a) {
     // only faces of this direction are ever flagged; the test keeps the stencil in range
     if (b >= g.nb || i < il || i > g.ie + 1 || j < jl || j > g.je + 1 || k < kl || k > g.ke + 1) continue;
     const int cidx = dir == 0 ? i : (dir == 1 ? j : k);
-    flux_face<ORDER, RS, float, ISO, false>(g, a, dir, b, id, cidx);
+    if (dir == 0) flux_face<0, ORDER, RS, float, ISO, false>(g, a, b, id, cidx);
+    else if (dir == 1) flux_face<1, ORDER, RS, float, ISO, false>(g, a, b, id, cidx);
+    else flux_face<2, ORDER, RS, float, ISO, false>(g, a, b, id, cidx);
   }
 }
 
@@ -3257,6 +3281,7 @@ int agx_calculate_fluxes(agx_mesh *m, int order) {
 }
 
 extern "C++" {
+constexpr int64_t LLC_BYTES = 256 << 20;   // last-level cache
 // k_flux in the directions dir0 .. dir0 + ndir - 1; FP32 PPM adds the k_flux_fix pass over the
 // faces k_flux flagged
 template <int ORD, int RS, typename TW, bool ISO>
@@ -3283,6 +3308,9 @@ static void launch_flux(agx_mesh *m, int dir0, int ndir) {
   a.gamma = m->d.gamma; a.cs = m->d.iso_cs; a.dfl = m->d.dfloor; a.pfl = m->d.pfloor;
   a.nearf = m->nearf; a.nflag = m->nearf_n;
   a.dir0 = dir0; a.ndir = ndir;
+  // w, bcc, the face fields read; fluxes, face EMFs and weights written (the mixed form keeps the
+  // latter 24 and w, bcc in FP32)
+  a.xcd = (int64_t)g.nb * g.S * (3 * 8 + 32 * (int64_t)sizeof(TW)) <= LLC_BYTES;
   // the largest plane of faces (x3: two more cells each way) and the most planes (x1, x2)
   const dim3 grid(ndir * grid1d((int64_t)(g.bx1 + 2) * (g.bx2 + 2), 256), (unsigned)(g.bx3 + 2), (unsigned)g.nb);
   hipLaunchKernelGGL((k_flux<ORD, RS, TW, ISO>), grid, dim3(256), 0, m->stream, g, a);

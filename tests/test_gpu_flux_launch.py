@@ -27,3 +27,22 @@ def test_directions_in_one_launch_identical(agx, bnx, order, precision):
         out.append([m.get(n) for n in ("u", "b1f", "b2f", "b3f")])
         m.close()
     assert all(np.array_equal(a, b) for a, b in zip(*out))
+
+
+@pytest.mark.parametrize("order,precision", [(1, 0), (2, 0), (3, 0), (2, 1), (3, 1)])
+def test_large_mesh_equals_one_launch_stage(agx, order, precision):
+    """arrays beyond the last-level cache, where k_flux takes its workgroups in plain order: the
+    split form against the stage that solves its faces itself"""
+    d = make_desc(nx=(128, 96, 100), bnx=(32, 24, 20), box=((0.0, 1.28), (0.0, 0.96), (0.0, 1.0)), cfl=0.3, nghost=3,
+                  xorder=order, precision=precision)
+    st = turbulent_state(d, seed=8, mach=2.0)
+    out = []
+    for form in (1, 5):
+        m = agx.Mesh(d)
+        load_state(m, st)
+        m.initialize()
+        m.set_tile(form)
+        m.cycle(1e9, 1)
+        out.append([m.get(n) for n in ("u", "b1f", "b2f", "b3f")])
+        m.close()
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
