@@ -2099,11 +2099,17 @@ __device__ __forceinline__ void flux_to_mesh(int dir, const T *f, T *out) {
   else { out[1] = f[2]; out[2] = f[3]; out[3] = f[1]; }
 }
 
+// the faces and the conserved state of a thread's cell while its update is formed
+struct CellUpdate {
+  double v3 = 0.0, b1l = 0.0, b1h = 0.0, b2l = 0.0, b2h = 0.0, un[NHYDRO];
+};
+
 template <int TI, int TJ, int ORDER, int RS, typename TW, bool ISO, bool PUSH>
 __global__ void __launch_bounds__(TI * TJ, 2)   // >= 2 waves per SIMD
 k_vl2(Geo g, VL2Args<TW> a, int kc) {
   static_assert(64 % TI == 0 && TI * TJ == 256, "k_vl2 tiles: 256 threads, rows within a wavefront");
-  constexpr bool EARLY = sizeof(TW) == 4;
+  constexpr bool EARLY = sizeof(TW) == 8 ? (ISO || RS == AGX_RSOLVER_HLLE)
+                                         : (ISO ? RS != AGX_RSOLVER_HLLE : RS != AGX_RSOLVER_ROE);
   constexpr int NH = ISO ? 4 : NHYDRO;
   constexpr int NT = TI * TJ;
   // current plane: x1 faces [ey=e3x1, ez=e2x1, w1][row jj+1][face ii]; x2 faces
@@ -2276,17 +2282,20 @@ k_vl2(Geo g, VL2Args<TW> a, int kc) {
         }
       }
     }
-    // the own column's loads and the conserved update of the cell of plane c-1.  FP32 runs them
-    // ahead of the barrier and of every store, as a load behind a store waits for it too (cycles of
-    // 128^3 PLM 2000 -> 1955 us); FP64, which has no registers for it, where they are used (ahead of the
-    // barrier 256^3 PLM took 9.6 ms a cycle instead of 9.2).
-    double v3 = 0.0, b1l = 0.0, b1h = 0.0, b2l = 0.0, b2h = 0.0, un[NHYDRO];
-    const bool cell = own && c - 1 >= kb;
-    auto load_faces = [&]() {
+    // the own column's loads and the conserved update of the cell of plane c-1: ahead of the barrier and
+    // of every store (EARLY), as a load behind a store waits for it too, where the 10 to 14 registers
+    // that stay live over the barrier neither spill nor cost a wave.  Cycles in us, where they are used :
+    // early, 256^3 in 64^3 blocks, PLM: FP32 HLLD 6889 : 6698, LHLLD 9427 : 9298, HLLE 7509 : 7373, Roe 7963 :
+    // 8083 (250 registers), isothermal HLLD 5998 : 5749, HLLE 5316 : 5603 (3 waves a SIMD : 2); FP64 HLLD 9162 :
+    // 9457, LHLLD 10864 : 11359, Roe 15768 : 17135 (each at 256 registers), HLLE 8601 : 8492, isothermal HLLD
+    // 8316 : 8051, HLLE 7543 : 7345.
+    CellUpdate early;
+    auto load_faces = [&](CellUpdate &q) __attribute__((always_inline)) {
       const int64_t fo = fb + IDX(g, c - 1, j, i);
-      b1l = a.s1[fo]; b1h = a.s1[fo + 1]; b2l = a.s2[fo]; b2h = a.s2[fo + sj];
+      q.b1l = a.s1[fo]; q.b1h = a.s1[fo + 1]; q.b2l = a.s2[fo]; q.b2h = a.s2[fo + sj];
     };
-    auto update_cell = [&]() {
+    auto update_cell = [&](CellUpdate &q) __attribute__((always_inline)) {
+      double *un = q.un;
       const int64_t id = IDX(g, c - 1, j, i);
       const int64_t fo = fb + id, cb0 = cbase + id;
       un[IEN] = 0.0;
@@ -2324,10 +2333,12 @@ k_vl2(Geo g, VL2Args<TW> a, int kc) {
       }
     };
     if constexpr (EARLY) {
-      if (own && c >= kb) v3 = a.s3[fb + IDX(g, c, j, i)];
-      if (cell) {
-        load_faces();
-        update_cell();
+      if (own && c >= kb) {
+        early.v3 = a.s3[fb + IDX(g, c, j, i)];
+        if (c - 1 >= kb) {
+          load_faces(early);
+          update_cell(early);
+        }
       }
     }
     __syncthreads();
@@ -2336,8 +2347,7 @@ k_vl2(Geo g, VL2Args<TW> a, int kc) {
     if (own && c >= kb) {
       {
         const int64_t fo = fb + IDX(g, c, j, i);
-        if constexpr (!EARLY) v3 = a.s3[fo];
-        double v = v3;
+        double v = EARLY ? early.v3 : a.s3[fo];
         const double area = dx1 * dx2;
         v -= (wght / area) * (dx2 * s_e2[cb][ty][tx + 1] - dx2 * s_e2[cb][ty][tx]);
         v += (wght / area) * (dx1 * s_e1[cb][ty + 1][tx] - dx1 * s_e1[cb][ty][tx]);
@@ -2351,11 +2361,14 @@ k_vl2(Geo g, VL2Args<TW> a, int kc) {
           for_each_ghost(g, b, c, j, i, r, [&](int nb, int64_t id2) { a.d3[(int64_t)nb * S + id2] = v; });
         }
       }
-      if (cell) {
+      if (c - 1 >= kb) {
         const int64_t id = IDX(g, c - 1, j, i);
         const int64_t fo = fb + id;
         const double area1 = dx2 * dx3, area2 = dx1 * dx3;
-        if constexpr (!EARLY) load_faces();
+        CellUpdate late;
+        CellUpdate &q = EARLY ? early : late;
+        if constexpr (!EARLY) load_faces(q);
+        double &b1l = q.b1l, &b1h = q.b1h, &b2l = q.b2l, &b2h = q.b2h, *un = q.un;
         b1l -= (wght / area1) * (dx3 * s_e3[pb][ty + 1][tx] - dx3 * s_e3[pb][ty][tx]);
         b1l += (wght / area1) * (dx2 * s_e2[cb][ty][tx] - dx2 * s_e2[pb][ty][tx]);
         b1h -= (wght / area1) * (dx3 * s_e3[pb][ty + 1][tx + 1] - dx3 * s_e3[pb][ty][tx + 1]);
@@ -2391,7 +2404,7 @@ k_vl2(Geo g, VL2Args<TW> a, int kc) {
           }
         }
         const int64_t cb0 = cbase + id;
-        if constexpr (!EARLY) update_cell();
+        if constexpr (!EARLY) update_cell(q);
         const double bcc1 = 0.5 * b1l + 0.5 * b1h;
         const double bcc2 = 0.5 * b2l + 0.5 * b2h;
         const double bcc3 = 0.5 * b3_lo + 0.5 * b3_hi;

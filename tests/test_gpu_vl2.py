@@ -4,7 +4,7 @@ bit.  Both forms form every value with the same operations in the same order, so
 array must be identical bit for bit after whole cycles: all Riemann solvers and
 reconstruction orders, both tile shapes, both EOS, FP64 and the mixed form, with
 self-gravity, on ragged MeshBlocks (tiles cut by the block edge) and on blocks smaller
-than a tile."""
+than a tile, and on meshes whose workgroups walk several k-planes of their own."""
 import numpy as np
 import pytest
 
@@ -56,6 +56,15 @@ CASES = [
      dict(mach=1.5, iso=True)),
     ("iso_hlle", dict(nx=(32, 32, 32), bnx=(16, 16, 16), box=((0, 1),) * 3, cfl=0.4, eos=1, iso_cs=0.8, rsolver=1),
      dict(mach=1.5, iso=True)),
+] + [
+    # chunks of several k-planes, the last one shorter (k_vl2: 4, 4, .., 2): what a workgroup carries
+    # from one of its planes to the next, in every solver and either place of the cell's update
+    (f"chunks_{name}", dict(nx=(72, 72, 66), bnx=(24, 24, 22), box=((0, 0.72), (0, 0.72), (0, 0.66)), cfl=0.4, **kw),
+     dict(mach=1.5, iso="eos" in kw))
+    for name, kw in (("hlld", {}), ("hlle", dict(rsolver=1)), ("roe", dict(rsolver=2)), ("lhlld", dict(rsolver=3)),
+                     ("dc", dict(xorder=1)), ("ppm", dict(xorder=3, nghost=3)), ("iso_hlld", dict(eos=1, iso_cs=0.8)),
+                     ("iso_hlle", dict(eos=1, iso_cs=0.8, rsolver=1)))
+] + [
     ("floors", dict(nx=(16, 16, 16), bnx=(8, 8, 8), box=((0, 1),) * 3, cfl=0.3),
      dict(p0=1e-19, vamp=0.3, drho=0.5)),
 ]
@@ -75,12 +84,15 @@ def test_one_launch_stage_equals_split(agx, name, dk, sk, precision):
 
 
 @pytest.mark.parametrize("precision", [0, 1])
-def test_one_launch_stage_with_self_gravity(agx, precision):
-    desc = make_desc(nx=(32, 32, 32), bnx=(16, 16, 16), box=((0, 1),) * 3, cfl=0.4, self_gravity=1,
-                     four_pi_G=1.0, mg_mode=0, mg_threshold=1e-9, precision=precision, xorder=3, nghost=3)
-    st = turbulent_state(desc, seed=21, mach=1.5, drho=0.5)
-    ref = run(agx, desc, st, 1, phi=True)
-    got = run(agx, desc, st, 5, phi=True)
+@pytest.mark.parametrize("n,b,eos", [(32, 16, 0), (128, 32, 0), (128, 32, 1)])   # one plane a workgroup; several
+def test_one_launch_stage_with_self_gravity(agx, n, b, eos, precision):
+    desc = make_desc(nx=(n,) * 3, bnx=(b,) * 3, box=((0, 1),) * 3, cfl=0.4, self_gravity=1,
+                     four_pi_G=1.0, mg_mode=0, mg_threshold=1e-9, precision=precision, xorder=3 if n == 32 else 2, nghost=3,
+                     eos=eos, iso_cs=0.8)
+    st = turbulent_state(desc, seed=21, mach=1.5, drho=0.5, iso=bool(eos))
+    ncyc = 3 if n == 32 else 1
+    ref = run(agx, desc, st, 1, ncyc, phi=True)
+    got = run(agx, desc, st, 5, ncyc, phi=True)
     assert got["time"] == ref["time"]
     for f in FIELDS + ("phi",):
         same(got[f], ref[f], f"self-gravity precision {precision}: {f}")
