@@ -159,14 +159,21 @@ static dim3 stage_grid(const Geo &g, int tile) {
 }
 
 // The form of a stage of reconstruction order `order` before any autotuning: the one launch
-// over 32 x 8 tiles, or the split form where that is faster: for PPM, whose faces cost
-// most (k_vl2 solves a quarter of them twice), and on meshes so small that k_vl2 would run chunks of
-// one or two planes (twice the work and more).  Cycles in us, k_vl2 against split: 64 x 32 x 32
-// 148 : 117, 64^3 in 32^3 blocks 263 : 236, 128^3 in 32^3 1369 : 1859 (FP64 PLM);
-// 120 x 90 x 70 in 40 x 30 x 14 blocks 1491 : 890 (FP64 PPM), 128^3 in 64^3 1692 : 1280 (mixed PPM).
-// Split tiles: 32 x 8 where it fits the rows (17 .. 32 cells), else 64 x 4.
+// over 32 x 8 tiles, or the split form where that is faster.  Cycles in us, k_vl2 against split, FP64 HLLD
+// PLM : mixed, unless it says otherwise:
+// - PPM, whose faces cost most (k_vl2 solves a quarter of them twice): the second stage alone split
+//   against both in k_vl2, 256^3 in 64^3 blocks 12045 : 13620 FP64, 8220 : 11950 mixed;
+// - meshes so small that k_vl2 would run chunks of one or two planes (twice the work and more):
+//   64 x 32 x 32 148 : 95 (mixed 120 : 83), 64^3 in 32^3 blocks 264 : 205 (198 : 161), but 96^3 742 : 743
+//   (530 : 568), 128^3 1363 : 1681 (977 : 1276), 256^3 in 64^3 9190 : 10450 (6717 : 6695).
+// Split tiles: 32 x 8 where it fits the rows (17 .. 32 cells), else 64 x 4; rows of at most 16 leave three
+// quarters of that idle, which costs nothing while its workgroups of one plane each are fewer than the
+// 1024 that the chip holds, and beyond 16 x 16 is faster (64 x 4 : 16 x 16, 16^3 blocks: 8 of them 92 : 100,
+// 12 107 : 114, 16 138 : 121, 32 215 : 152, 64 390 : 281; 12^3: 16 of them 100 : 94, 32 143 : 112; 64^3 in 8^3
+// 840 : 656; PPM 64^3 in 16^3 520 : 391).
 static int default_form(const Geo &g, int order) {
-  const int split = (g.bx1 > 16 && g.bx1 <= 32) ? 1 : 2;
+  const int64_t wg64 = (int64_t)stage_tiles(g, 2) * g.nb * g.bx3;
+  const int split = g.bx1 <= 16 ? (wg64 < 1024 ? 2 : 0) : (g.bx1 <= 32 ? 1 : 2);
   return (order == 3 || stage_planes(g, 5) <= 2) ? split : 5;
 }
 
