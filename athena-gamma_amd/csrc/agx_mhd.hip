@@ -165,16 +165,18 @@ static dim3 stage_grid(const Geo &g, int tile) {
 //   against both in k_vl2, 256^3 in 64^3 blocks 12045 : 13620 FP64, 8220 : 11950 mixed;
 // - meshes so small that k_vl2 would run chunks of one or two planes (twice the work and more):
 //   64 x 32 x 32 148 : 95 (mixed 120 : 83), 64^3 in 32^3 blocks 264 : 205 (198 : 161), but 96^3 742 : 743
-//   (530 : 568), 128^3 1363 : 1681 (977 : 1276), 256^3 in 64^3 9190 : 10450 (6717 : 6695).
+//   (530 : 568), 128^3 1363 : 1681 (977 : 1276), 256^3 in 64^3 9190 : 10450 (6717 : 6695);
+// - FP64 Roe (roe64), whose k_vl2 spills 178 registers: 256^3 in 64^3 15760 : 11710, 128^3 in 32^3
+//   2250 : 1776, 200 x 120 x 96 2960 : 1574.
 // Split tiles: 32 x 8 where it fits the rows (17 .. 32 cells), else 64 x 4; rows of at most 16 leave three
 // quarters of that idle, which costs nothing while its workgroups of one plane each are fewer than the
 // 1024 that the chip holds, and beyond 16 x 16 is faster (64 x 4 : 16 x 16, 16^3 blocks: 8 of them 92 : 100,
 // 12 107 : 114, 16 138 : 121, 32 215 : 152, 64 390 : 281; 12^3: 16 of them 100 : 94, 32 143 : 112; 64^3 in 8^3
 // 840 : 656; PPM 64^3 in 16^3 520 : 391).
-static int default_form(const Geo &g, int order) {
+static int default_form(const Geo &g, int order, bool roe64) {
   const int64_t wg64 = (int64_t)stage_tiles(g, 2) * g.nb * g.bx3;
   const int split = g.bx1 <= 16 ? (wg64 < 1024 ? 2 : 0) : (g.bx1 <= 32 ? 1 : 2);
-  return (order == 3 || stage_planes(g, 5) <= 2) ? split : 5;
+  return (order == 3 || roe64 || stage_planes(g, 5) <= 2) ? split : 5;
 }
 
 template <typename X>
@@ -2788,9 +2790,10 @@ int agx_mesh_create(const agx_mesh_desc *desc, agx_mesh **out) {
   g.PL = g.PL > g.n3 ? g.PL : g.n3;
   g.J = g.n2 + 1;
   g.S = (int64_t)(g.n3 + 1) * g.J * g.P;
-  m->tile1 = default_form(g, 1);
+  const bool roe64 = desc->rsolver == AGX_RSOLVER_ROE && desc->precision != AGX_PREC_MIXED;
+  m->tile1 = default_form(g, 1, roe64);
   // characteristic projection is built into the split forms only: 32 x 8 for its stage
-  m->tile = (m->d.char_proj && m->d.xorder > 1) ? 1 : default_form(g, m->d.xorder);
+  m->tile = (m->d.char_proj && m->d.xorder > 1) ? 1 : default_form(g, m->d.xorder, roe64);
   // variables per array: the AGX_ARR_* set, then W2, BCC2, Q1F, Q2F, Q3F
   static const int nv[ARR_TOTAL] = {5, 5, 5, 3, 1, 1, 1, 1, 1, 1, 5, 5, 5,
                                     1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1,

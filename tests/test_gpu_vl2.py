@@ -96,3 +96,22 @@ def test_one_launch_stage_with_self_gravity(agx, n, b, eos, precision):
     assert got["time"] == ref["time"]
     for f in FIELDS + ("phi",):
         same(got[f], ref[f], f"self-gravity precision {precision}: {f}")
+
+
+@pytest.mark.parametrize("rsolver,precision,split", [(0, 0, False), (2, 0, True), (2, 1, False)])
+def test_default_form_of_roe(agx, rsolver, precision, split):
+    """FP64 Roe, whose one-launch stage spills, starts in the split form on a mesh where the others
+    start in the one launch; either gives the other's arrays"""
+    desc = make_desc(nx=(96, 96, 96), bnx=(32, 32, 32), box=((0, 1),) * 3, cfl=0.4, rsolver=rsolver, precision=precision)
+    st = turbulent_state(desc, seed=19, mach=1.5)
+    m = agx.Mesh(desc)
+    load_state(m, st)
+    m.initialize()
+    m.timing(True)
+    m.cycle(1e9, 1)
+    assert (m.timing_get("flux_x1")[1] > 0) == split
+    got = {f: m.get(f) for f in FIELDS}
+    m.close()
+    ref = run(agx, desc, st, 5 if split else 1, 1)
+    for f in FIELDS:
+        same(got[f], ref[f], f"rsolver {rsolver} precision {precision}: {f}")
