@@ -70,6 +70,27 @@ k_mg_smooth(const int *__restrict__ gate, T *__restrict__ u, const T *__restrict
   u[id] = gs_value(uc, ukp, ujp, uip, ukm, ujm, uim, src[id], dx2, isix);
 }
 
+// The sweep of a level with an odd extent of three or more, where the periodic wrap joins cells of
+// one colour: out of place, so that every update reads the values from before the sweep, as the
+// reference's do from ghosts filled ahead of it.  In place the value read across the wrap would be
+// whichever of old and new another workgroup has stored.  Only a root grid's lowest level is odd.
+template <typename T>
+__global__ void __launch_bounds__(BS)
+k_mg_smooth_wrap(const int *__restrict__ gate, const T *__restrict__ u, T *__restrict__ out, const T *__restrict__ src,
+                 int n1, int n2, int n3, T dx2, T isix, int color) {
+  if (gate && *gate) return;   // a closed gate: the recorded V-cycle loop has ended
+  const unsigned t = blockIdx.x * BS + threadIdx.x;
+  if (t >= (unsigned)n1 * n2 * n3) return;
+  const unsigned r = t / (unsigned)n1;
+  const int i = (int)(t - r * n1), j = (int)(r % (unsigned)n2), k = (int)(r / (unsigned)n2);
+  T v = u[t];
+  if (((color + i + j + k) & 1) == 0)
+    v = gs_value(v, u[LIX(n1, n2, wrapp(k, n3), j, i)], u[LIX(n1, n2, k, wrapp(j, n2), i)],
+                 u[LIX(n1, n2, k, j, wrapp(i, n1))], u[LIX(n1, n2, wrapm(k, n3), j, i)],
+                 u[LIX(n1, n2, k, wrapm(j, n2), i)], u[LIX(n1, n2, k, j, wrapm(i, n1))], src[t], dx2, isix);
+  out[t] = v;
+}
+
 // The same red/black sweep with one thread per (i, i+1) pair of a row (n1 even): the
 // pair is read and written as one 16-B (8-B in FP32) vector, so rows are read and
 // written as whole cache lines; the cell of the pair that is not of this colour is
@@ -2662,8 +2683,13 @@ static void smooth(agx_mesh *m, std::vector<MGLevelT<T>> &H, int l, int color) {
   double dx2 = L.dx * L.dx;
   double isix = 1.15 / 6.0;
   int64_t n = (int64_t)((L.n1 + 1) / 2) * L.n2 * L.n3;
+  auto odd = [](int q) { return (q & 1) && q > 1; };
   timer_begin(m, AGX_K_MG_SMOOTH);
-  if ((L.n1 & 1) == 0)
+  if (odd(L.n1) || odd(L.n2) || odd(L.n3)) {
+    hipLaunchKernelGGL(k_mg_smooth_wrap<T>, dim3(grid1d(lcells(L), BS)), dim3(BS), 0, m->stream, m->gate, L.u, L.def,
+                       L.src, L.n1, L.n2, L.n3, T(dx2), T(isix), color ^ m->coffset);
+    std::swap(L.u, L.def);
+  } else if ((L.n1 & 1) == 0)
     hipLaunchKernelGGL(k_mg_smooth_pairs<T>, dim3(grid1d(n, BS)), dim3(BS), 0, m->stream, m->gate, L.u, L.src, L.n1,
                        L.n2, L.n3, T(dx2), T(isix), color ^ m->coffset);
   else
