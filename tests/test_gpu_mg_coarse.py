@@ -1,7 +1,9 @@
 """k_mg_coarse, k_mg_down and k_mg_up against the per-level steps at the edges of their ranges: the
 whole hierarchy in the coarse kernel (16^3 cells, and one 8^3 block), root grids that are odd or
-flat, levels just above it, levels of one tile, of several and of parts of one, flat ones, and
-chunks that end inside; the same potential bit for bit."""
+flat, levels just above it, levels of one tile, of several and of parts of one, and flat ones; chunks
+of two planes (the small shapes), of eight (128^3), and of six with a last one of four (192 x 160 x 40,
+the finest level of one shape and a level with a FAS right-hand side of another); the same potential
+bit for bit."""
 import numpy as np
 import pytest
 
@@ -11,7 +13,8 @@ from tests.test_gpu_mg_levels import vcycle_by_steps
 pytestmark = pytest.mark.gpu
 
 SHAPES = [((8, 8, 8), 8), ((16, 16, 16), 8), ((24, 8, 8), 8), ((12, 20, 4), 4), ((64, 8, 4), 4), ((32, 32, 32), 8),
-          ((40, 24, 56), 8), ((72, 16, 8), 8), ((96, 48, 16), 16), ((128, 128, 4), 4)]
+          ((40, 24, 56), 8), ((72, 16, 8), 8), ((96, 48, 16), 16), ((128, 128, 4), 4), ((128, 128, 128), 32),
+          ((192, 160, 40), 8), ((384, 320, 80), 16)]
 
 
 @pytest.mark.parametrize("precision", [0, 1])
@@ -60,7 +63,7 @@ def test_periodic_vcycle_identical(agx, n, b):
 
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("n,b", [((40, 24, 56), 8), ((64, 64, 64), 32), ((128, 32, 32), 32), ((128, 128, 4), 4),
-                                 ((96, 48, 16), 16), ((36, 20, 12), 4)])
+                                 ((96, 48, 16), 16), ((36, 20, 12), 4), ((128, 128, 128), 32), ((192, 160, 40), 8)])
 def test_periodic_passes_identical(agx, n, b, precision):
     """whole passes against one launch per step"""
     h = 1.0 / max(n)
