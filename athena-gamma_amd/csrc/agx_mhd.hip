@@ -1364,12 +1364,15 @@ __device__ __forceinline__ void flux_face(const Geo &g, const FluxArgs<T> &a, in
   if constexpr (FLAG) a.nearf[dir * a.nflag + fo] = near ? 1 : 0;
 }
 
-// Waves per SIMD asked of the compiler: FP64 characteristic PLM takes 176 registers, 2 waves, where
-// 168 with four spilled are 3 (256^3 in 64^3 blocks: 3.54 ms a launch, as three launches took); Roe and
-// LHLLD would spill 20 to 106.
-template <int ORDER, int RS, typename T>
+// Waves per SIMD asked of the compiler where three directions in one kernel take a few registers
+// more than a count allows (FP64; 1: no bound).  Characteristic PLM: 176 registers, 2 waves, where 168
+// with four spilled are 3 (256^3 in 64^3 blocks 3.54 ms a launch, as three launches took); Roe and LHLLD
+// would spill 20 to 106.  HLLE: PPM 104 and isothermal PLM 97, 4 waves, where 96 are 5.
+template <int ORDER, int RS, typename T, bool ISO>
 constexpr int flux_waves() {
-  return ORDER == ORDER_PLM_CHAR && sizeof(T) == 8 && (RS == AGX_RSOLVER_HLLD || RS == AGX_RSOLVER_HLLE) ? 3 : 1;
+  if (sizeof(T) != 8) return 1;
+  if (ORDER == ORDER_PLM_CHAR) return RS == AGX_RSOLVER_HLLD || RS == AGX_RSOLVER_HLLE ? 3 : 1;
+  return RS == AGX_RSOLVER_HLLE && (ORDER == 3 || (ORDER == 2 && ISO)) ? 5 : 1;
 }
 
 // Hydro::CalculateFluxes, one thread per face (face_flux), the directions of the launch in one
@@ -1391,7 +1394,7 @@ constexpr int flux_waves() {
 // For FP32 PPM nearf (one byte per cell of the block arrays and direction) receives each face's
 // near-tie flag.
 template <int ORDER, int RS, typename T, bool ISO>
-__global__ void __launch_bounds__(256, (flux_waves<ORDER, RS, T>()))
+__global__ void __launch_bounds__(256, (flux_waves<ORDER, RS, T, ISO>()))
 k_flux(Geo g, FluxArgs<T> a) {
   const uint3 wg = a.xcd ? xcd_block() : make_uint3(blockIdx.x, blockIdx.y, blockIdx.z);
   const int part = (int)(wg.x / (unsigned)a.ndir), dir = a.dir0 + (int)(wg.x - part * (unsigned)a.ndir);
