@@ -358,29 +358,16 @@ __device__ __forceinline__ void wg_range(unsigned n, unsigned &t0, unsigned &t1)
   if (t0 > n) t0 = n;
 }
 
-// block-partial sums in FP64: mode 0 sum(a), mode 1 sum(def^2)
-template <int MODE, typename T>
+// block-partial sums of a level array in FP64
+template <typename T>
 __global__ void __launch_bounds__(BS)
-k_mg_partial(const int *__restrict__ gate, const T *__restrict__ a, const T *__restrict__ src, int n1, int n2, int n3,
-             T idx2, double *__restrict__ part) {
+k_mg_partial(const int *__restrict__ gate, const T *__restrict__ a, unsigned ncell, double *__restrict__ part) {
   if (gate && *gate) return;   // a closed gate: the recorded V-cycle loop has ended
   __shared__ double sh[BS];
-  const unsigned ncell = (unsigned)n1 * n2 * n3;   // < 2^32 cells per level
   unsigned t0, t1;
-  wg_range(ncell, t0, t1);
+  wg_range(ncell, t0, t1);   // < 2^32 cells per level
   double v = 0.0;
-  for (unsigned t = t0 + threadIdx.x; t < t1; t += BS) {
-    if (MODE == 0) {
-      v += a[t];
-    } else {
-      int i = (int)(t % (unsigned)n1);
-      unsigned r = t / (unsigned)n1;
-      int j = (int)(r % (unsigned)n2);
-      int k = (int)(r / (unsigned)n2);
-      double d = defect_at(a, src, n1, n2, n3, k, j, i, idx2);
-      v += d * d;
-    }
-  }
+  for (unsigned t = t0 + threadIdx.x; t < t1; t += BS) v += a[t];
   sh[threadIdx.x] = v;
   __syncthreads();
   for (int s = BS / 2; s > 0; s >>= 1) {
@@ -390,10 +377,10 @@ k_mg_partial(const int *__restrict__ gate, const T *__restrict__ a, const T *__r
   if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
-// k_mg_partial's mode 1 with a thread's cells as (i, i+1) pairs of a row (n1 even), read as one
-// vector, and stepped from pair to pair without divisions, which were most of its instructions:
-// 256^3 FP64 93 -> 66 us, 4.0 TB/s of u and source.  Each thread sums its own pairs, so the order
-// differs from mode 1's, which runs where n1 is odd.
+// block-partial sums of the squared defect, a thread's cells as (i, i+1) pairs of a row read as one
+// vector and stepped from pair to pair without divisions, which were most of the instructions of a
+// cell at a time: 256^3 FP64 93 -> 66 us, 4.0 TB/s of u and source.  For the finest level, whose rows
+// are even (a MeshBlock has at least two cells along i, a power of two).
 template <typename T>
 __global__ void __launch_bounds__(BS)
 k_mg_norm_pairs(const int *__restrict__ gate, const T *__restrict__ u, const T *__restrict__ src, int n1, int n2,
@@ -2221,7 +2208,7 @@ static void vcycle_b(agx_mesh *m) {
   const Geo &g0 = m->g;
   const int ct = coarse_top_b(m);
   if (ct >= 0) {
-    // the levels above the coarse kernel's range launch per step; from level
+    // the levels above the coarse kernel's range as whole passes, or per step where they are flat; from level
     // min(start, ct) down to 0 and back, one launch
     while (m->current > ct) {
       const int l = m->current;
@@ -2612,7 +2599,7 @@ int mg_create(agx_mesh *m) {
       int64_t n = pad32(lcells(Lv));
       Lv.u = q; q += n;
       Lv.src = q; q += n;
-      Lv.def = q; q += n;   // spare array of the fused red-black pass
+      Lv.def = q; q += n;   // spare array (whole passes, the mixed correction)
     }
   }
   int64_t need = (lcells(m->lev[L - 1]) + BS - 1) / BS + 1;
@@ -2731,33 +2718,29 @@ static void fmg_prolong(agx_mesh *m, std::vector<MGLevelT<T>> &H, int l) {   // 
   timer_end(m);
 }
 
-// device sum of a level array (mode 0) or of its squared defect (mode 1) into scal[slot]
+// device sum of a level array into scal[slot]
 template <typename T>
-static void level_sum(agx_mesh *m, std::vector<MGLevelT<T>> &H, int l, int mode, int slot) {
-  MGLevelT<T> &L = H[l];
-  int64_t nb = npart(lcells(L));
-  double idx2 = 1.0 / (L.dx * L.dx);
-  timer_begin(m, AGX_K_MG_OTHER);
-  if (mode == 0)
-    hipLaunchKernelGGL((k_mg_partial<0, T>), dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, L.u, L.src, L.n1,
-                       L.n2, L.n3, T(idx2), m->red);
-  else if ((L.n1 & 1) == 0) {
-    nb = npart(lcells(L) / 2);
-    hipLaunchKernelGGL(k_mg_norm_pairs<T>, dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, L.u, L.src, L.n1,
-                       L.n2, L.n3, T(idx2), m->red);
-  } else
-    hipLaunchKernelGGL((k_mg_partial<1, T>), dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, L.u, L.src, L.n1,
-                       L.n2, L.n3, T(idx2), m->red);
+static void array_sum(agx_mesh *m, const MGLevelT<T> &L, const T *a, int slot) {
+  const int64_t nb = npart(lcells(L));
+  hipLaunchKernelGGL(k_mg_partial<T>, dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, a, (unsigned)lcells(L),
+                     m->red);
   final_sum(m, nb, slot);
+}
+template <typename T>
+static void level_sum(agx_mesh *m, std::vector<MGLevelT<T>> &H, int l, int slot) {
+  timer_begin(m, AGX_K_MG_OTHER);
+  array_sum(m, H[l], H[l].u, slot);
   timer_end(m);
 }
-
-static void level_sum_src(agx_mesh *m, int l, int slot) {
-  MGLevel &L = m->lev[l];
-  int64_t nb = npart(lcells(L));
-  hipLaunchKernelGGL((k_mg_partial<0, double>), dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, L.src, L.src,
-                     L.n1, L.n2, L.n3, 0.0, m->red);
-  final_sum(m, nb, slot);
+// the finest FP64 level's squared defect into scal[0]
+static void defect_sum(agx_mesh *m) {
+  MGLevel &L = m->lev[m->ntotal - 1];
+  const int64_t nb = npart(lcells(L) / 2);
+  timer_begin(m, AGX_K_MG_OTHER);
+  hipLaunchKernelGGL(k_mg_norm_pairs<double>, dim3((unsigned)nb), dim3(BS), 0, m->stream, m->gate, L.u, L.src, L.n1,
+                     L.n2, L.n3, 1.0 / (L.dx * L.dx), m->red);
+  final_sum(m, nb, 0);
+  timer_end(m);
 }
 
 static double mesh_volume(const agx_mesh_desc &d) {
@@ -2772,8 +2755,8 @@ static void subtract_average(agx_mesh *m, int type) {
   MGLevel &L = m->lev[l];
   const agx_mesh_desc &d = m->d;
   double dv = m->rdx_blk * m->rdy_blk * m->rdz_blk;
-  if (type == 0) level_sum_src(m, l, 1);
-  else level_sum(m, m->lev, l, 0, 1);
+  if (type == 0) array_sum(m, L, L.src, 1);
+  else level_sum(m, m->lev, l, 1);
   double scale = dv / mesh_volume(d);
   hipLaunchKernelGGL(k_mg_add<double>, dim3(grid1d(lcells(L), BS)), dim3(BS), 0, m->stream, m->gate,
                      type ? L.u : L.src, lcells(L), m->scal + 1, scale);
@@ -2808,7 +2791,7 @@ static void solve_coarsest(agx_mesh *m, std::vector<MGLevelT<T>> &H) {
     if (pass == 1) {
       for (int it = 0; it < ni; ++it) { smooth(m, H, 0, 0); smooth(m, H, 0, 1); }
     }
-    level_sum(m, H, 0, 0, 2);
+    level_sum(m, H, 0, 2);
     hipLaunchKernelGGL(k_mg_add<T>, dim3(grid1d(lcells(LR), BS)), dim3(BS), 0, m->stream, m->gate, LR.u, lcells(LR),
                        m->scal + 2, scale);
   }
@@ -2922,7 +2905,7 @@ static double finish_norm(agx_mesh *m) {
 
 static double defect_norm(agx_mesh *m) {
   // MultigridDriver::CalculateDefectNorm (L2), multigrid_driver.cpp:826-858
-  level_sum(m, m->lev, m->ntotal - 1, 1, 0);
+  defect_sum(m);
   return finish_norm(m);
 }
 
@@ -3014,7 +2997,7 @@ static int retrieve(agx_mesh *m) {
 static void first_defect_sum(agx_mesh *m) {
   if (m->mp_on) defect_sum_b(m);
   else if (m->mixed) defect_to32(m, false);
-  else level_sum(m, m->lev, m->ntotal - 1, 1, 0);
+  else defect_sum(m);
 }
 static void loop_step(agx_mesh *m) {
   if (m->mp_on) {
@@ -3025,7 +3008,7 @@ static void loop_step(agx_mesh *m) {
     correction_step(m);   // the defect comes with the correction
   } else {
     vcycle(m, m->lev);
-    level_sum(m, m->lev, m->ntotal - 1, 1, 0);
+    defect_sum(m);
   }
 }
 
@@ -3289,7 +3272,7 @@ int mg_vcycles(agx_mesh *m, int n) {
 // The multigrid at the granularity of the reference's MultigridTaskList
 // (multigrid/mg_task_list.cpp:183-280, 287-530) and MGGravity / Multigrid methods, on
 // the FP64 hierarchy (every level of the whole mesh, finest = nlevels - 1), for callers
-// that drive their own cycles.  They use the same kernels as agx_mg_solve, so a V(1,1)
+// that drive their own cycles.  Each value is formed by the arithmetic of agx_mg_solve's whole passes, so a V(1,1)
 // cycle composed of them equals agx_mg_vcycles(1) bit for bit.
 static int mg_level_check(agx_mesh *m, int level, int lo, const char *who) {
   if (!m) { set_error("%s: null mesh", who); return -1; }

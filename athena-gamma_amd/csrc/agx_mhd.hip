@@ -95,19 +95,15 @@ struct PlaneIdx {
 };
 
 // (b,k,j,i) of this thread for the box [kl..ku]x[jl..ju]x[il..iu]; false if outside.
-// With xcd, workgroups are taken in the XCD-aware order (xcd_block): consecutive planes
-// of a block then run on one XCD, which pays off for kernels with a k stencil.
-__device__ __forceinline__ bool plane_index(int il, int iu, int jl, int ju, int kl, PlaneIdx &p,
-                                            bool xcd = false) {
+__device__ __forceinline__ bool plane_index(int il, int iu, int jl, int ju, int kl, PlaneIdx &p) {
   const unsigned ni = iu - il + 1, nj = ju - jl + 1;
-  const uint3 wg = xcd ? xcd_block() : make_uint3(blockIdx.x, blockIdx.y, blockIdx.z);
-  const unsigned q = wg.x * blockDim.x + threadIdx.x;
+  const unsigned q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= ni * nj) return false;
   const unsigned qj = q / ni;
   p.j = jl + (int)qj;
   p.i = il + (int)(q - qj * ni);
-  p.k = kl + (int)wg.y;
-  p.b = wg.z;
+  p.k = kl + (int)blockIdx.y;
+  p.b = blockIdx.z;
   return true;
 }
 
@@ -4090,7 +4086,7 @@ int agx_autotune(agx_mesh *m, int32_t *choice) {
 
 int agx_set_mg_fuse(agx_mesh *m, int32_t mode) {
   if (!m) { set_error("null mesh"); return -1; }
-  if (mode < -1 || mode > 1) { set_error("red-black pass form %d not in {-1, 0, 1}", mode); return -2; }
+  if (mode < -1 || mode > 1) { set_error("multigrid pass form %d not in {-1, 0, 1}", mode); return -2; }
   m->mg_fuse = mode;
   m->graph_gen++;
   return 0;

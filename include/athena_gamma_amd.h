@@ -302,8 +302,10 @@ int agx_block_gids(const agx_mesh_desc *d, int64_t *lattice_of_gid);
  * 34-40; Multigrid::Restrict/ProlongateAndCorrect/FMGProlongate, multigrid.hpp:120-127)
  * for callers that drive their own cycles.  Each step runs on one level of the FP64
  * hierarchy of the whole mesh (level 0 = root, agx_mg_levels gives the count and sizes)
- * with the kernels of agx_mg_solve, so a V(1,1) composed of them equals agx_mg_vcycles(1)
- * bit for bit.  Order of a V(1,1) from the finest level F, after agx_mg_coffset(m, 1, 0):
+ * with the arithmetic of agx_mg_solve, so a V(1,1) composed of them equals agx_mg_vcycles(1)
+ * bit for bit.  (agx_mg_solve and agx_mg_vcycles run whole passes of a level and leave on the
+ * levels below the finest what those need; begin a cycle of steps with agx_mg_setup, or continue
+ * the finest level's potential.)  Order of a V(1,1) from the finest level F, after agx_mg_coffset(m, 1, 0):
  *   periodic:  l = F..1: smooth(l,0), smooth(l,1), restrict(l); solve_coarsest;
  *              l = 1..F: prolong(l), smooth(l,0), smooth(l,1)
  *   multipole: l = F..1: fill_ghost(l), [fas(l) if l < F], smooth(l,0), fill_ghost(l),
@@ -330,11 +332,11 @@ int agx_mg_levels(agx_mesh *m, int32_t *nlevels, int32_t *dims, int32_t cap);
 /* ---- tuning (no counterpart in the reference: launch shapes of this library).
  * agx_autotune times each form of a VL2 stage on the current state, for the first
  * (donor-cell) stage and for the second (the mesh's order) separately, and keeps the
- * fastest for each; *choice gets the second stage's form.  Forms 0..3: three flux launches, then one stage
+ * fastest for each; *choice gets the second stage's form.  Forms 0..3: one launch for the fluxes, then one stage
  * kernel over 16x16, 32x8, 64x4 (i,j) columns per 256-thread workgroup or 64x8 per
  * 512-thread workgroup; forms 4..5: the whole stage (fluxes in LDS) in one launch over
- * 16x16 or 32x8 columns.  Without autotuning each stage runs form 5, or on small meshes and
- * for PPM a split form.  With multigrid
+ * 16x16 or 32x8 columns.  Without autotuning each stage runs form 5, or on small meshes, for PPM
+ * and for Roe in FP64 a split form.  With multigrid
  * gravity (periodic boundaries) it also times V-cycles with whole passes of a level (both
  * sweeps and the transfer in one launch) and with one launch per step, and keeps the faster.  It writes only scratch registers
  * (u1, b1, fluxes, the multigrid levels, which every solve reloads), so call it between
@@ -611,7 +613,12 @@ int agx_device_alloc(int64_t bytes, void **out);
 int agx_device_free(void *p);
 int agx_device_copy(void *dst, const void *src, int64_t bytes, int32_t kind);
 
-/* ---- built-in timers (HIP events on the mesh stream around each launch) */
+/* ---- built-in timers (HIP events on the mesh stream around each launch).  While they are on, cycles
+ * run eagerly, the fluxes of a split stage run as one launch per direction (one for all three
+ * otherwise), and threshold solves read the norm after every V-cycle.  AGX_K_MG_SMOOTH holds whole
+ * passes of a level (sweeps, FAS right-hand side and transfer in one launch) and the periodic coarse
+ * levels, AGX_K_MG_OTHER the multipole ones; AGX_K_MG_RESTRICT and AGX_K_MG_PROLONG the transfers that
+ * run by themselves: FMG, and cycles with one launch per step. */
 int agx_timing_enable(agx_mesh *m, int enable);
 int agx_timing_reset(agx_mesh *m);
 int agx_timing_get(agx_mesh *m, int kclass, double *ms_total, int64_t *launches);

@@ -108,7 +108,7 @@ def test_source_mask_matches(agx, bc):
 @pytest.mark.parametrize("mode,thr,nit", [(0, -1.0, 3), (0, 0.0, 0), (1, -1.0, 2)])
 @pytest.mark.parametrize("precision", [0, 1])
 def test_coarse_kernel_identical(agx, mode, thr, nit, precision):
-    """the coarse end of the multipole V-cycle in one workgroup (k_mb_coarse) against one
+    """the coarse end of the multipole V-cycle in one workgroup (k_mg_coarse) against one
     launch per step: the same potential bit for bit (FMG + fixed cycles, threshold 0,
     MGI), on a 4x2x2 root grid of 16^3 blocks; FP64, and the mixed form, whose FP32
     correction cycles use the kernel's homogeneous-boundary FP32 instance"""

@@ -66,9 +66,8 @@ def test_absolute_threshold_iterations():
 
 
 def test_fused_red_black_levels():
-    """FP64 levels of >= 2^26 cells run both sweeps of each red-black pass in one launch
-    (k_mg_smooth_rb); 512 x 512 x 256 in MeshBlocks of 256^3 is the smallest such mesh
-    with a cubic-MeshBlock hierarchy.  Fixed V-cycle counts: the oracle's iterate
+    """A finest level of 2^26 cells, which k_mg_down and k_mg_up walk in one chunk of all its
+    planes: 512 x 512 x 256 in MeshBlocks of 256^3.  Fixed V-cycle counts: the oracle's iterate
     sequence, same bar."""
     agx = load_agx()
     N1, N3, B = 512, 256, 256
@@ -107,10 +106,9 @@ def test_fused_red_black_levels():
 
 @pytest.mark.parametrize("precision", [0, 1])
 def test_red_black_pass_forms_identical(precision):
-    """The fused red-black pass (one launch, k_mg_smooth_rb) and two sweeps give the same
-    potential bit for bit, in FP64 and in the FP32 correction cycles of the mixed form;
-    128^3 is the smallest mesh whose finest level (2^21 cells) the forced fused form
-    covers.  The autotuner picks one of the two, so its choice cannot change results."""
+    """Whole passes of a level (k_mg_down, k_mg_up) and one launch per step give the same
+    potential bit for bit, in FP64 and in the FP32 correction cycles of the mixed form.  The
+    autotuner picks one of the two, so its choice cannot change results."""
     agx = load_agx()
     N, B = 128, 32
     d = make_desc(nx=(N, N, N), bnx=(B, B, B), box=((0, 1),) * 3, self_gravity=1, mg_mode=0,
@@ -128,7 +126,7 @@ def test_red_black_pass_forms_identical(precision):
         out.append(m.get("phi"))
         m.close()
     d_ = np.abs(out[0] - out[1]).max()
-    print(f"precision {precision}: max |phi(two sweeps) - phi(fused)| = {d_:.3e}", flush=True)
+    print(f"precision {precision}: max |phi(steps) - phi(passes)| = {d_:.3e}", flush=True)
     assert np.array_equal(out[0], out[1])
 
 

@@ -1,5 +1,5 @@
-"""The one-launch VL2 stage (k_vl2: fluxes in LDS) against the split form (three flux
-launches + the stage kernel), which the other parity tests hold to the oracle bit for
+"""The one-launch VL2 stage (k_vl2: fluxes in LDS) against the split form (the flux
+launch + the stage kernel), which the other parity tests hold to the oracle bit for
 bit.  Both forms form every value with the same operations in the same order, so every
 array must be identical bit for bit after whole cycles: all Riemann solvers and
 reconstruction orders, both tile shapes, both EOS, FP64 and the mixed form, with
@@ -75,7 +75,7 @@ CASES = [
 def test_one_launch_stage_equals_split(agx, name, dk, sk, precision):
     desc = make_desc(precision=precision, **dk)
     st = turbulent_state(desc, seed=17, **sk)
-    ref = run(agx, desc, st, 1)          # k_flux x 3 + k_stage<32, 8>
+    ref = run(agx, desc, st, 1)          # k_flux + k_stage<32, 8>
     for tile in (4, 5):                  # k_vl2<16, 16>, k_vl2<32, 8>
         got = run(agx, desc, st, tile)
         assert got["time"] == ref["time"]
