@@ -102,6 +102,12 @@ def max_divb(desc, m):
     return dmax, dmax * min(dx) / float(bmax)
 
 
+# Multigrid, bytes per finest cell of a periodic V(1,1) whose levels run as whole passes, all levels (8/7):
+# down reads u and the source and writes u and an eighth of the coarse source and u (26 B in FP64), up reads
+# u, the source and an eighth of the coarse u and writes u (25 B).  A mixed correction cycle: the same in FP32
+# and 36 B for the FP64 defect and correction (phi, e and source read; phi, FP32 source and e written).
+PASS_BYTES = {"fp64": 51.0 * 8.0 / 7.0, "mixed": 25.5 * 8.0 / 7.0}
+VCYCLE_BYTES = {"fp64": PASS_BYTES["fp64"], "mixed": PASS_BYTES["mixed"] + 36.0}
 KCLASSES = ("flux_x1", "flux_x2", "flux_x3", "corner_e", "integrate", "bvals", "c2p", "newdt")
 
 
@@ -347,11 +353,11 @@ def sg_run(agx, pgen, N, B, xorder, mach, steps, tag, bx=None, sensitivity=False
         per = {c: m.timing_get(c) for c in KCLASSES + ("mg_smooth", "mg_restrict", "mg_prolong", "mg_other")}
         m.timing(False)
         # whole-cycle byte model: the MHD cycle (680 B FP64 / 552 B mixed per zone) and two
-        # solves, each load + FMG (about 8/7 of a finest-level V-cycle) + vc V-cycles at
-        # 148.6 B (FP64) or 114.3 B (mixed correction cycle) per zone, + retrieve (16 B)
+        # solves, each load + FMG (8/7 of a V-cycle of plain passes) + vc V-cycles with the norm
+        # (mixed: correction cycles, which form it) + retrieve (16 B)
         key = "mixed" if prec == "mixed" else "fp64"
-        vbytes = 114.3 if key == "mixed" else 148.6
-        bcyc = CYCLE_BYTES[key] + 2 * (24.0 + vbytes * (8.0 / 7.0 + vc) + 16.0)
+        fmg = PASS_BYTES[key] * 8.0 / 7.0
+        bcyc = CYCLE_BYTES[key] + 2 * (24.0 + fmg + (VCYCLE_BYTES[key] + (16.0 if key == "fp64" else 0.0)) * vc + 16.0)
         res[prec] = dict(zc=float(N) ** 3 * steps / sec, ms=sec * 1e3 / steps, w=w, bcc=bcc, phi=phi, divb=divb,
                          per=per, tile=tile, bytes=m.device_bytes(), vc=vc, bcyc=bcyc,
                          rf=roofline(desc, per, key, tile))
@@ -937,7 +943,7 @@ def main():
     if not args.no_mg:
         vps, iters, norm, t_solve, mper = mg_bench(agx, pgen, args)
         out["mg_vcycles_per_s"] = vps
-        out["mg_roofline_frac"] = vps * float(args.n) ** 3 * 148.6 / HBM_PEAK
+        out["mg_roofline_frac"] = vps * float(args.n) ** 3 * VCYCLE_BYTES["fp64"] / HBM_PEAK
         out["mg_solve_ms_to_1e-10"] = t_solve * 1e3
         out["mg_solve_vcycles_after_fmg"] = iters
         out["mg_kernel_ms_per_vcycle"] = {k: v[0] / 3 for k, v in mper.items()}
@@ -946,7 +952,7 @@ def main():
             out["mg_mixed"] = {
                 "vcycles_per_s": vps32, "vs_fp64": vps32 / vps,
                 "note": "one cycle = FP64 defect + FP32 V(1,1) + FP64 correction",
-                "roofline_frac": vps32 * float(args.n) ** 3 * 114.3 / HBM_PEAK,
+                "roofline_frac": vps32 * float(args.n) ** 3 * VCYCLE_BYTES["mixed"] / HBM_PEAK,
                 "solve_ms_to_1e-10": ts32 * 1e3, "cycles_after_fmg": it32, "final_defect": norm32,
                 "kernel_ms_per_cycle": {k: v[0] / 3 for k, v in mper32.items()}}
         vmp, itmp, nmp, tsmp, mpper = mg_bench(agx, pgen, args, "multipole")
