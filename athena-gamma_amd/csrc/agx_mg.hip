@@ -1340,10 +1340,10 @@ k_mg_coarse(const int *__restrict__ gate, CoarseSet<T> S, int top, int fmglevel,
 // steps staggered: red on plane q, black on q-1, the defect on q-2.  A colour's update is one
 // cell of every pair, so no lane idles; its neighbours along k are the thread's own registers,
 // those along i and j come from the plane in LDS, updated in place.  The steps of an iteration
-// work on different planes, and one barrier a plane suffices.  256^3 FP64 periodic: 133 us down
-// (two sweeps and the restriction: 238) and 136 us up (263), where the bytes of u and source
+// work on different planes, and one barrier a plane suffices.  256^3 FP64 periodic: 126 us down
+// (two sweeps and the restriction: 238) and 130 us up (263), where the bytes of u and source
 // alone take 80; 64^3 multipole: 14 us down and 12 up (29 and 32 with the ghost fills).  On
-// large levels an iteration's instructions bound it (about 300 for a pair of cells and a plane,
+// large levels an iteration's instructions bound it (259 down and 198 up for a pair of cells,
 // 44 of them floating point), on small ones their latency: loads two or three planes ahead and
 // planes split by cell parity in LDS made it no faster.  A tile held whole in LDS takes the same
 // time on small levels and 36 us instead of 34 at 128^3.
