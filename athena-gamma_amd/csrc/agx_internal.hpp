@@ -122,7 +122,7 @@ struct MGLevelB32 {
 
 // Device state of a threshold solve whose V-cycle loop is recorded for a fixed number of
 // passes (the graph replay of agx_cycle).  While closed != 0 every multigrid kernel of the
-// loop returns at once; k_mg_gate_check closes it where SolveIterative's loop stops.
+// loop returns at once; k_mg_final_check closes it where SolveIterative's loop stops.
 struct MGGate {
   int closed;
   int iters;     // V-cycles the loop has run
